@@ -203,39 +203,55 @@ struct MisArgs {
 
 // ------------------------------------------------------- spanning forest
 // One run of pbbs_spanning_forest (st.hip).  The control words of the round
-// schedule (common/speculative_for.h:30-100) live in device memory.
-struct StCtl {
-  long long done;          // iterations finished (numberDone)
-  long long nkeep;         // failed iterates carried to the front of this round
+// schedule (common/speculative_for.h:30-100) live in device memory, in two
+// slots: round r's reserve kernel reads slot r & 1 (the round before) and
+// writes the other one.
+struct StSlot {
+  long long done;          // iterations finished (numberDone) when the round began
+  long long nkeep;         // failed iterates carried to the front of the round
   long long cur;           // currentRoundSize
-  long long size;          // this round's iterates
-  long long scatter_size;  // the round just scheduled, for its pack kernel (0: none)
-  long long rounds;        // rounds scheduled so far
+  long long size;          // the round's iterates
+  long long rounds;        // rounds completed before it
+  int finished;
+  int pad;
+};
+
+struct StCtl {
+  StSlot slot[2];
+  long long rounds;        // rounds completed
   long long count;         // forest edges, after the output scan
   int error;               // bits: 1 an edge end outside [0, n), 2 the schedule gave up,
                            // 4 an any-forest edge ran out of tries
-  int finished;
+  int filter;              // tree_bits holds a tree's vertices
 };
 
-constexpr int kStMaxGroups = 4096;   // workgroups of a round launch at most
+constexpr int kStMaxGroups = 4096;   // workgroups of an output launch at most
 constexpr int kStScanPer = 4;        // counts each thread of the one-workgroup scan sums
+constexpr int kStMaxTiles = 1024;    // tiles of a round (one workgroup each) at most
 
 struct StArgs {
   const int32_t* eu;       // [m] edge ends
   const int32_t* ev;
   int32_t* parents;        // [n] union-find, -1 at roots
   uint32_t* R;             // [n] reservations, UINT_MAX when free
-  uint32_t* I;             // [max_round] this round's iterates
-  int32_t* su;             // [max_round] their roots, su < sv
+  unsigned long long* tree_bits;   // [ceil(n / 64)] vertices known to lie in the large tree
+  // per tile of the round, a.tile entries each: the iterates whose ends lie in
+  // different trees, with their roots su < sv, and the losers among them
+  uint32_t* I;
+  int32_t* su;
   int32_t* sv;
-  uint8_t* keep;           // [max_round] reserved and not yet committed
-  uint32_t* hold[2];       // [max_round] failed iterates, by round parity
-  unsigned* blk;           // [kStMaxGroups] per-workgroup counts, then offsets
+  uint32_t* hold;
+  unsigned* cand;          // [kStMaxTiles] entries of I, su, sv
+  unsigned* lost;          // [kStMaxTiles] entries of hold
+  unsigned* blk;           // [kStMaxGroups] per-workgroup counts of the output, then offsets
   StCtl* ctl;
   int32_t* host_status;    // pinned: [0] done, [1] rounds
   long long n, m;
   long long max_round;     // m / granularity + 1
   long long max_tries;     // 100 + 200 * granularity
+  long long tile;          // iterates per tile, a multiple of step * kBlock
+  int step;                // iterates per thread and step: 1, 4 or 8
+  int pad;
 };
 
 }  // namespace pbbs

@@ -63,7 +63,8 @@ template <typename OffT>
 hipError_t launch_mis_output(const MisArgs<OffT>& a, int32_t* flags_out,
                              unsigned long long* members, int grid, hipStream_t stream);
 hipError_t launch_st_init(const StArgs& a, int grid, hipStream_t stream);
-hipError_t launch_st_round(const StArgs& a, int grid, hipStream_t stream);
+hipError_t launch_st_round(const StArgs& a, long long round, int grid, hipStream_t stream);
+hipError_t launch_st_tree(const StArgs& a, long long round, int grid, hipStream_t stream);
 hipError_t launch_st_any(const StArgs& a, int grid, hipStream_t stream);
 hipError_t launch_st_output(const StArgs& a, int32_t* forest, int grid, hipStream_t stream);
 template <typename OffT>
@@ -224,15 +225,16 @@ struct pbbs_ctx {
   unsigned long long* s_ctl = nullptr;   // kMisCtlWords
   unsigned long long* s_part = nullptr;  // kMaxGrid
   uint32_t* s_wg = nullptr;              // kMaxGrid
-  // spanning forest: union-find and reservations per vertex, the round's
-  // iterates and their roots, the two carry lists, per-workgroup counts, the
-  // schedule's control words, and the edges when the caller's are in host
-  // memory
+  // spanning forest: union-find, reservations and the large tree's bitmap per
+  // vertex, the round's iterates, their roots and the losers, per-tile and
+  // per-workgroup counts, the schedule's control words, and the edges when the
+  // caller's are in host memory
   int64_t cap_tn = 0, cap_tr = 0, cap_te = 0;
   int32_t* t_parents = nullptr;
   uint32_t* t_R = nullptr;
-  unsigned char* t_round = nullptr;      // I | su | sv | hold0 | hold1 | keep
-  unsigned* t_blk = nullptr;
+  unsigned long long* t_bits = nullptr;
+  uint32_t* t_round = nullptr;           // I | su | sv | hold, cap_tr entries each
+  unsigned* t_blk = nullptr;             // blk | cand | lost
   StCtl* t_ctl = nullptr;
   int32_t* t_edges = nullptr;            // eu | ev, cap_te each
   int32_t* t_out = nullptr;              // cap_tn forest entries for a host copy
@@ -312,9 +314,12 @@ constexpr int kMisCtlWords = kMisCtlMembers + 8;
 
 static int64_t mis_region(int64_t n) { return (n + kMisStripes - 1) / kMisStripes + kMisMaxChunk; }
 
+constexpr int kStCounts = kStMaxGroups + 2 * kStMaxTiles;
+
 static void free_st_workspace(pbbs_ctx* c) {
   (void)hipFree(c->t_parents);
   (void)hipFree(c->t_R);
+  (void)hipFree(c->t_bits);
   (void)hipFree(c->t_round);
   (void)hipFree(c->t_blk);
   (void)hipFree(c->t_ctl);
@@ -322,14 +327,15 @@ static void free_st_workspace(pbbs_ctx* c) {
   (void)hipFree(c->t_out);
   c->t_parents = c->t_out = c->t_edges = nullptr;
   c->t_R = nullptr;
+  c->t_bits = nullptr;
   c->t_round = nullptr;
   c->t_blk = nullptr;
   c->t_ctl = nullptr;
   c->cap_tn = c->cap_tr = c->cap_te = 0;
 }
 
-// Grows the spanning-forest workspace to n vertices, r iterates a round and
-// (host edges) e edges; buffers only grow.
+// Grows the spanning-forest workspace to n vertices, r iterates over a round's
+// tiles and (host edges) e edges; buffers only grow.
 static int ensure_st_workspace(pbbs_ctx* c, int64_t n, int64_t r, int64_t e) {
   if (n <= c->cap_tn && r <= c->cap_tr && e <= c->cap_te && c->t_ctl) return PBBS_OK;
   const int64_t cn = std::max(n, c->cap_tn), cr = std::max(r, c->cap_tr),
@@ -338,8 +344,9 @@ static int ensure_st_workspace(pbbs_ctx* c, int64_t n, int64_t r, int64_t e) {
   if (hipMalloc(&c->t_parents, std::max<int64_t>(cn, 1) * sizeof(int32_t)) != hipSuccess ||
       hipMalloc(&c->t_R, std::max<int64_t>(cn, 1) * sizeof(uint32_t)) != hipSuccess ||
       hipMalloc(&c->t_out, std::max<int64_t>(cn, 1) * sizeof(int32_t)) != hipSuccess ||
-      hipMalloc(&c->t_round, std::max<int64_t>(cr, 1) * 21) != hipSuccess ||
-      hipMalloc(&c->t_blk, kStMaxGroups * sizeof(unsigned)) != hipSuccess ||
+      hipMalloc(&c->t_bits, (cn + 63) / 64 * sizeof(unsigned long long)) != hipSuccess ||
+      hipMalloc(&c->t_round, std::max<int64_t>(cr, 1) * 4 * sizeof(uint32_t)) != hipSuccess ||
+      hipMalloc(&c->t_blk, kStCounts * sizeof(unsigned)) != hipSuccess ||
       hipMalloc(&c->t_ctl, sizeof(StCtl)) != hipSuccess ||
       (ce > 0 && hipMalloc(&c->t_edges, 2 * ce * sizeof(int32_t)) != hipSuccess)) {
     (void)hipGetLastError();
@@ -1341,6 +1348,13 @@ extern "C" int pbbs_mis(pbbs_ctx* c, pbbs_graph* g, int32_t* flags, uint32_t out
 // The round schedule's constants for granularity 100 (spanningForest/
 // incrementalST/ST.C:69; common/speculative_for.h:33-38).
 constexpr int64_t kStGranularity = 100;
+// The large tree's bitmap pays where `parents` (4 bytes a vertex) outgrows an
+// XCD's 4 MB L2.  It is written before round 8 (about 3% of the edges in, when
+// the tree first holds enough of an RMAT graph: first rounds 6, 8, 10 and 12
+// measured 5.85, 5.81, 5.82 and 5.79 ms on 190.6M edges) and again at every
+// half as many rounds more (twice as many: 5.88 ms).
+constexpr int64_t kStTreeVertices = int64_t(1) << 20;
+constexpr int64_t kStFirstTree = 8;
 
 extern "C" int pbbs_spanning_forest(pbbs_ctx* c, int64_t n, int64_t m, const int32_t* u,
                                     const int32_t* v, uint32_t flags, int32_t* forest,
@@ -1362,22 +1376,29 @@ extern "C" int pbbs_spanning_forest(pbbs_ctx* c, int64_t n, int64_t m, const int
                 (long long)m, (long long)(3 * kStGranularity));
   HIP_TRY(hipSetDevice(c->device));
   const bool dev_edges = (flags & PBBS_EDGES_DEVICE) != 0;
-  int rc = ensure_st_workspace(c, n, max_round, dev_edges ? 0 : m);
-  if (rc != PBBS_OK) return rc;
   StArgs a{};
   a.n = n;
   a.m = m;
+  // one iterate per thread while the tiles can be that small; beyond, more
+  // loads in flight per thread
+  a.step = max_round <= kStMaxTiles * kBlock ? 1 : max_round <= 4 * kStMaxTiles * kBlock ? 4 : 8;
+  const int64_t per_step = (int64_t)a.step * kBlock;
+  a.tile = (max_round + kStMaxTiles * per_step - 1) / (kStMaxTiles * per_step) * per_step;
+  const int64_t tiles = (max_round + a.tile - 1) / a.tile;   // of the largest round
+  int rc = ensure_st_workspace(c, n, tiles * a.tile, dev_edges ? 0 : m);
+  if (rc != PBBS_OK) return rc;
   a.max_round = max_round;
   a.max_tries = 100 + 200 * kStGranularity;
   a.parents = c->t_parents;
   a.R = c->t_R;
-  a.I = reinterpret_cast<uint32_t*>(c->t_round);
-  a.su = reinterpret_cast<int32_t*>(c->t_round + 4 * c->cap_tr);
-  a.sv = reinterpret_cast<int32_t*>(c->t_round + 8 * c->cap_tr);
-  a.hold[0] = reinterpret_cast<uint32_t*>(c->t_round + 12 * c->cap_tr);
-  a.hold[1] = reinterpret_cast<uint32_t*>(c->t_round + 16 * c->cap_tr);
-  a.keep = c->t_round + 20 * c->cap_tr;
+  a.tree_bits = c->t_bits;
+  a.I = c->t_round;
+  a.su = reinterpret_cast<int32_t*>(c->t_round + c->cap_tr);
+  a.sv = reinterpret_cast<int32_t*>(c->t_round + 2 * c->cap_tr);
+  a.hold = c->t_round + 3 * c->cap_tr;
   a.blk = c->t_blk;
+  a.cand = c->t_blk + kStMaxGroups;
+  a.lost = a.cand + kStMaxTiles;
   a.ctl = c->t_ctl;
   a.host_status = c->host_status;
   double copy_ms = 0.0;
@@ -1395,11 +1416,6 @@ extern "C" int pbbs_spanning_forest(pbbs_ctx* c, int64_t n, int64_t m, const int
     }
     HIP_TRY(hipEventRecord(c->ev_c1, c->stream));
   }
-  // round launches: one thread per iterate of the largest round, up to
-  // kStMaxGroups workgroups (the finds are chains of dependent loads, so
-  // more of them in flight is what hides their latency)
-  const int64_t tiles = (max_round + kBlock - 1) / kBlock;
-  const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(tiles, kStMaxGroups));
   const int init_grid = (int)std::min<int64_t>(std::max<int64_t>((n + kBlock - 1) / kBlock, 1),
                                                8 * c->num_cus);
   volatile int32_t* hs = c->host_status;
@@ -1409,6 +1425,7 @@ extern "C" int pbbs_spanning_forest(pbbs_ctx* c, int64_t n, int64_t m, const int
   // size), so the first chunk launches that many; then chunks of 8
   const int64_t limit = a.max_tries + 2;
   int64_t launched = 0;
+  int64_t next_tree = n > kStTreeVertices ? kStFirstTree : limit;   // the round it precedes
   int K = (int)std::min<int64_t>(std::max<int64_t>((m + max_round - 1) / max_round, 8), limit);
   if (any) {   // one pass over the edges, no schedule
     const int any_grid = (int)std::min<int64_t>(std::max<int64_t>((m + kBlock - 1) / kBlock, 1),
@@ -1418,7 +1435,13 @@ extern "C" int pbbs_spanning_forest(pbbs_ctx* c, int64_t n, int64_t m, const int
   }
   for (; K > 0;) {
     const int k = (int)std::min<int64_t>(K, limit - launched);
-    for (int i = 0; i < k; ++i) HIP_TRY(launch_st_round(a, grid, c->stream));
+    for (int i = 0; i < k; ++i) {
+      if (launched + i == next_tree) {
+        HIP_TRY(launch_st_tree(a, next_tree, init_grid, c->stream));
+        next_tree += next_tree / 2;
+      }
+      HIP_TRY(launch_st_round(a, launched + i, (int)tiles, c->stream));
+    }
     launched += k;
     HIP_TRY(hipEventRecord(c->ev_end, c->stream));
     HIP_TRY(hipEventSynchronize(c->ev_end));
@@ -1429,7 +1452,9 @@ extern "C" int pbbs_spanning_forest(pbbs_ctx* c, int64_t n, int64_t m, const int
     K = 8;
   }
   int32_t* d_out = (flags & PBBS_OUT_DEVICE) && forest ? forest : c->t_out;
-  HIP_TRY(launch_st_output(a, d_out, grid, c->stream));
+  const int out_grid =
+      (int)std::min<int64_t>(std::max<int64_t>((n + kBlock - 1) / kBlock, 1), kStMaxGroups);
+  HIP_TRY(launch_st_output(a, d_out, out_grid, c->stream));
   StCtl hc{};
   HIP_TRY(hipMemcpyAsync(&hc, c->t_ctl, sizeof hc, hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipEventRecord(c->ev_end, c->stream));
@@ -1933,7 +1958,9 @@ int64_t ctx_workspace_bytes(const pbbs_ctx* c) {
          2 * (int64_t)kSubQueues * c->cap_bn * 8;
   if (c->b_parent) b += 2 * c->cap_bout * 4;
   if (c->b_parent_alt) b += c->cap_bout * 4;
-  if (c->t_ctl) b += 12 * c->cap_tn + 21 * c->cap_tr + 8 * c->cap_te + kStMaxGroups * 4;
+  if (c->t_ctl)
+    b += 12 * c->cap_tn + (c->cap_tn + 63) / 64 * 8 + 16 * c->cap_tr + 8 * c->cap_te +
+         kStCounts * 4;
   if (c->s_flags)
     b += 9 * c->cap_sn + 8 * kMisStripes * mis_region(c->cap_sn) + kMisCtlWords * 8 +
          kMaxGrid * 12;
