@@ -108,6 +108,7 @@ struct BfsArgs {
   int32_t symmetric;
   int32_t num_cus;             // CUs of the device (workgroup slot = blockIdx / num_cus)
   int32_t small_rows;          // 1 if no row has more than 64 entries (top-down slices by entry)
+  unsigned long long* deep_words;  // meeting words of a deep launch to clear, or null
   long long wait_ticks;        // persistent launch: longest barrier wait (device wall-clock
                                // ticks) before the launch gives up
 };
@@ -116,6 +117,29 @@ struct BfsArgs {
 // own graph, in one launch): an array of their BfsArgs and the first
 // workgroup of each (njobs + 1 entries, the last one the grid size).
 constexpr int kMaxMultiJobs = 64;
+
+// --------------------------------------------------------- deep graphs
+// A persistent launch that meets every few levels (bfs_deep.hip).
+constexpr int kDeepBlock = 256;        // threads per workgroup
+constexpr int kDeepMaxGroups = 1024;   // workgroups at most
+constexpr int kDeepCap = 2048;         // frontier entries a workgroup holds
+constexpr int kDeepCand = 4096;        // neighbours it claims in a level
+constexpr int kDeepSeenBits = 12;      // log2 of the claimed vertices its filter holds
+constexpr int kDeepMaxRow = 64;        // entries of the longest row it takes
+constexpr int kDeepPhases = 64;        // levels between two meetings at most
+// A frontier up to kDeepSolo goes to one workgroup, which advances alone until
+// it holds more than kDeepSoloMax (64/128, 64/256, 128/256, 256/512 measured
+// 109, 110, 112, 190 us on the 18^3 torus and 1.559, 1.568, 1.561, 1.596 ms on
+// 216^3).
+constexpr int kDeepSolo = 64;
+constexpr int kDeepSoloMax = 128;
+constexpr int kDeepMaxParts = 2048;    // workgroups of the parents pass at most
+
+struct DeepWs {
+  unsigned long long* words;   // [2][kDeepMaxGroups] meeting words
+  unsigned long long* lists;   // [2][groups][kDeepCap] frontier entries
+  unsigned long long* part;    // [kDeepMaxParts][4] totals of the parents pass's workgroups
+};
 
 // ----------------------------------------------------------- batched BFS
 // Up to 64 sources in one traversal: bit i of a per-vertex 64-bit mask

@@ -33,27 +33,9 @@
 #include <rocprim/iterator/counting_iterator.hpp>
 
 #include "bfs_device.hpp"
+#include "gmem.hpp"
 
 namespace pbbs {
-
-// Device pointers typed in the global address space, so loads, stores and
-// atomics through them compile to global_* instructions.  Generic (flat)
-// accesses also count against the LDS counter, so every LDS or cross-lane
-// wait would otherwise wait for the outstanding memory loads too.
-#define PBBS_GLOBAL __attribute__((address_space(1)))
-template <typename T>
-using gptr = PBBS_GLOBAL T*;
-template <typename T>
-__device__ __forceinline__ gptr<T> glob(T* p) {
-  return (gptr<T>)p;
-}
-// Generic pointer for the atomic builtins; the compiler still sees the
-// global origin and emits global atomics.
-template <typename T>
-__device__ __forceinline__ T* gen(gptr<T> p) {
-  return (T*)p;
-}
-
 
 // ---------------------------------------------------------------- wave utils
 __device__ __forceinline__ unsigned lane_id() { return __lane_id(); }
@@ -1375,6 +1357,8 @@ __global__ __launch_bounds__(kBlock) void bfs_init_kernel(BfsArgs<OffT> a, BfsAr
     a.fb[2][w] = 0ull;
   }
   for (long long i = tid; i < kMaxGrid; i += nth) a.wg_level[i] = 0;
+  if (a.deep_words)
+    for (long long i = tid; i < 2 * kDeepMaxGroups; i += nth) a.deep_words[i] = 0;
   if (tid == 0) {
     BfsArgs<OffT> b = a;
     b.iso = iso;

@@ -41,6 +41,11 @@ template <typename OffT>
 hipError_t launch_bfs_persist(const BfsArgs<OffT>* dargs, int variant, int grid,
                               hipStream_t stream);
 template <typename OffT>
+const void* deep_kernel_symbol();
+template <typename OffT>
+hipError_t launch_bfs_deep(const BfsArgs<OffT>* dargs, const DeepWs& ws, bool sorted, int grid,
+                           int parents_grid, hipStream_t stream);
+template <typename OffT>
 hipError_t launch_graph_offsets(const OffT* off, long long n, long long m,
                                 unsigned long long* iso, unsigned long long* counters, int grid,
                                 hipStream_t stream);
@@ -181,6 +186,10 @@ struct pbbs_ctx {
     bool graphs = true;           // single source: captured launch graphs allowed (the
                                   // context's own workspace only; capture allocates)
   } run;
+  // deep graphs: meeting words, the parents pass's totals and frontier lists
+  // for d_groups workgroups (one allocation)
+  int d_groups = 0;
+  unsigned long long* d_deep = nullptr;
   // batched BFS
   int64_t cap_bn = 0;                    // vertices the mask buffers hold
   unsigned long long* b_masks = nullptr; // vis | fr0 | fr1 | fr2 | fr3
@@ -268,6 +277,8 @@ struct pbbs_graph {
   // Level launches the last single-source [0] / batched [1] run needed (its
   // levels plus the launch that found the frontier empty); 0 = none yet.
   std::atomic<int> last_launches[2] = {0, 0};
+  // A deep launch found the graph's frontiers too large for it: not tried again.
+  std::atomic<bool> not_deep{false};
 };
 
 // One persistent launch per device at a time: its grid fills the device and
@@ -300,6 +311,9 @@ static void free_workspace(pbbs_ctx* c) {
   (void)hipFree(c->w_qe);
   c->w_parent = c->w_depth = nullptr;
   c->w_bits = nullptr;
+  (void)hipFree(c->d_deep);
+  c->d_deep = nullptr;
+  c->d_groups = 0;
   c->w_q = nullptr;
   c->w_qe = nullptr;
   c->cap_n = 0;
@@ -1036,8 +1050,10 @@ static int poll_run_impl(pbbs_ctx* c, bool wait, bool* done) {
     r.persist = false;
     if (!c->host_status[2])
       return fail(PBBS_ERR_STATE, "persistent BFS launch ended before the BFS did");
-    // the launch gave up waiting at a barrier (the device was shared): run the
-    // BFS again from its start, one level per launch
+    if (c->host_status[2] == 2) r.graph->not_deep = true;
+    // the launch gave up waiting at a barrier (the device was shared), or the
+    // frontier outgrew the deep path: run the BFS again from its start, one
+    // level per launch
     return restart_levels(c);
   }
   if (r.launched > r.limit)
@@ -1101,6 +1117,56 @@ static bool want_persist(const pbbs_ctx* c, const pbbs_graph* g) {
   return g->last_launches[0] - 1 >= kPersistMinLevels;   // levels + 1 launches
 }
 
+// A persistent launch takes the deep path (bfs_deep.hip) on symmetric graphs
+// of short rows: most of what a level costs is then latency and the meeting of
+// the workgroups, which the deep path pays once every few levels.  It pays
+// from fewer levels on than the other persistent launch: the 24^3 torus, 37
+// levels, takes 329 us one level per launch and 125 so, 10^3 (16 levels) 145
+// and 84.  Its lists are allocated, so runs in a caller's block do without it;
+// and it leaves any-parent runs alone, whose bottom-up levels decide the
+// parents.
+constexpr int kDeepMinLevels = 16;
+
+static bool want_deep(const pbbs_ctx* c, const pbbs_graph* g, bool own, bool any_parent) {
+  if (!own || any_parent || !g->symmetric || g->max_degree > kDeepMaxRow || g->not_deep)
+    return false;
+  if (c->tuning.persist == 1) return true;
+  return c->tuning.persist == 2 && g->last_launches[0] - 1 >= kDeepMinLevels;
+}
+
+// The deep path's buffers for `groups` workgroups; false if there is no room
+// (the run then takes the other path).
+static bool ensure_deep(pbbs_ctx* c, int groups, DeepWs* ws) {
+  const size_t words = 2 * kDeepMaxGroups, part = 4 * kDeepMaxParts;
+  const size_t lists = (size_t)2 * groups * kDeepCap;
+  if (groups > c->d_groups) {
+    (void)hipFree(c->d_deep);
+    c->d_deep = nullptr;
+    c->d_groups = 0;
+    if (hipMalloc(&c->d_deep, (words + part + lists) * sizeof(unsigned long long)) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    c->d_groups = groups;
+  }
+  ws->words = c->d_deep;
+  ws->part = c->d_deep + words;
+  ws->lists = c->d_deep + words + part;
+  return true;
+}
+
+// Workgroups of the deep kernel: the tuning's grid_blocks if set, else two per
+// CU, never more than are resident at once.
+template <typename OffT>
+static int deep_grid(pbbs_ctx* c) {
+  int per_cu = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, deep_kernel_symbol<OffT>(),
+                                                   kDeepBlock, 0) != hipSuccess)
+    return 0;
+  const int want = c->tuning.grid_blocks > 0 ? c->tuning.grid_blocks : 2 * c->num_cus;
+  return std::min({want, per_cu * c->num_cus, kDeepMaxGroups});
+}
+
 // Starts a single-source BFS.  With allow_persist, every level runs in one
 // persistent launch when the tuning asks for it and this context can take
 // the device's token; otherwise the levels run one per launch, in captured
@@ -1118,8 +1184,16 @@ static int begin_bfs(pbbs_ctx* c, pbbs_graph* g, int32_t s, int32_t* d_parent, i
   if (rc != PBBS_OK) return rc;
   const int variant = any_parent ? kLevelAnyParent : level_variant(g, tops);
   int grid = level_grid(c, g->off64, variant);
-  bool persist = false;
-  if (allow_persist && want_persist(c, g)) {
+  bool persist = false, deep = false;
+  DeepWs dws{};
+  if (allow_persist && want_deep(c, g, own, any_parent)) {
+    const int dg = deep_grid<OffT>(c);
+    if (dg >= 1 && ensure_deep(c, dg, &dws) && take_persist(c)) {
+      persist = deep = true;
+      grid = dg;
+    }
+  }
+  if (allow_persist && !persist && want_persist(c, g)) {
     const int cap = persist_capacity(c, g->off64, variant);
     if (cap >= 1 && take_persist(c)) {
       persist = true;
@@ -1127,12 +1201,15 @@ static int begin_bfs(pbbs_ctx* c, pbbs_graph* g, int32_t s, int32_t* d_parent, i
     }
   }
   const uint32_t* bounds = nullptr;
-  rc = ensure_bounds(c, g, (int64_t)grid * kWavesPerBlock, &bounds, own);
-  if (rc != PBBS_OK) {
-    release_persist(c);
-    return rc;
+  if (!deep) {   // the deep path has no bottom-up levels
+    rc = ensure_bounds(c, g, (int64_t)grid * kWavesPerBlock, &bounds, own);
+    if (rc != PBBS_OK) {
+      release_persist(c);
+      return rc;
+    }
   }
   BfsArgs<OffT> a = make_args<OffT>(c, g, ws, d_parent, d_depth, bounds, tops);
+  a.deep_words = dws.words;
   const int init_grid =
       (int)std::max<int64_t>(1, std::min<int64_t>((g->n + kBlock - 1) / kBlock, c->num_cus * 16));
   pbbs_ctx::Run& r = c->run;
@@ -1164,6 +1241,13 @@ static int begin_bfs(pbbs_ctx* c, pbbs_graph* g, int32_t s, int32_t* d_parent, i
   if (!restart) HIP_TRY(hipEventRecord(c->ev_start, c->stream));
   HIP_TRY(launch_bfs_init<OffT>(a, static_cast<BfsArgs<OffT>*>(ws.args), g->d_iso, s, init_grid,
                                 c->stream));
+  if (deep) {
+    HIP_TRY(launch_bfs_deep<OffT>(static_cast<const BfsArgs<OffT>*>(ws.args), dws, g->sorted, grid,
+                                  std::min(init_grid, kDeepMaxParts), c->stream));
+    r.launched = 1;
+    HIP_TRY(hipEventRecord(c->ev_end, c->stream));
+    return PBBS_OK;
+  }
   if (persist) {
     HIP_TRY(launch_bfs_persist<OffT>(static_cast<const BfsArgs<OffT>*>(ws.args), variant, grid,
                                      c->stream));
@@ -1956,6 +2040,7 @@ int64_t ctx_workspace_bytes(const pbbs_ctx* c) {
   if (c->b_masks)
     b += 5 * c->cap_bn * 8 + 4 * bwords * 8 + c->cap_bn * kMaxSources +
          2 * (int64_t)kSubQueues * c->cap_bn * 8;
+  if (c->d_deep) b += (2 * kDeepMaxGroups + 4 * kDeepMaxParts + (int64_t)2 * c->d_groups * kDeepCap) * 8;
   if (c->b_parent) b += 2 * c->cap_bout * 4;
   if (c->b_parent_alt) b += c->cap_bout * 4;
   if (c->t_ctl)
