@@ -198,29 +198,50 @@ struct MbfsArgs {
 };
 
 // ------------------------------------------------- maximal independent set
-// One run of pbbs_mis (mis.hip): flags[v] 0 undecided, 1 in the set, 2 out;
-// pos[v] the row position the next look at v starts from (written when v is
-// deferred, read in later rounds only).  A round's deferred vertices go to
-// kMisStripes regions of the next list, `region` entries each, with a count
-// per region: three sets of counts rotate (ctr + set * kMisStripes * 16, one
-// count per 128-byte line), so no one address takes every append.
+// One run of pbbs_mis (mis.hip): two bits per vertex say it is in the set or
+// out of it (neither: undecided); pos[v] the row position the next look at v
+// starts from (written when v is deferred, read in later rounds only).  A
+// round's deferred vertices go to kMisStripes regions of the next list,
+// `region` entries each, with a count per region: three sets of counts rotate
+// (ctr + set * kMisStripes * 16, one count per 128-byte line), so no one
+// address takes every append.
 constexpr int kMisStripes = 64;
 constexpr int kMisMaxChunk = 1024;   // list entries one wavefront takes at a time
+constexpr int kMisPer = 4;           // fresh vertices a lane looks at together
+constexpr int kMisRetry = 1;         // second looks at a list chunk's deferred vertices
+constexpr int kMisSmall = 16384;     // vertices up to which one workgroup runs it all
+constexpr int kMisSmallBlock = 1024;
+constexpr int kAdjPad = 4;           // entries past a graph's last that may be read
+
+// First vertex of round r's block: the first three rounds take an eighth, a
+// quarter and a half of a block (with no vertex decided yet, most first looks
+// would be blocked), the others `block` vertices, up to n.
+constexpr long long mis_block_start(long long block, long long n, int r) {
+  const long long e = block / 8;
+  const long long at = r <= 3 ? e * ((1ll << r) - 1) : e * 7 + (r - 3) * block;
+  return at < n ? at : n;
+}
+
+// {in, out} word pairs of 32 vertices, two pairs for every 64.
+constexpr long long mis_state_words(long long n) { return (n + 63) / 64 * 2; }
 
 template <typename OffT>
 struct MisArgs {
   const OffT* off;
   const int32_t* adj;
-  uint8_t* flags;              // [n]
+  unsigned long long* state;   // [mis_state_words(n)] in (low 32 bits) and out of 32 vertices
   uint32_t* pos;               // [n] relative to the row start
   int32_t* list[2];            // [kMisStripes * region] each
   unsigned long long* ctr;     // [3][kMisStripes][16]
   unsigned long long* part;    // [kMaxGrid] set members per output workgroup
   uint32_t* wg_round;          // kMaxGrid per-workgroup round counters
   int32_t* finished;
-  int32_t* host_status;        // pinned: [0] done, [1] rounds started
+  int32_t* host_status;        // pinned: [0] done, [1] rounds started, [2] a region overflowed,
+                               // [4..5] set members
   int64_t n;
-  int64_t region;              // entries per list region: ceil(n / kMisStripes) + kMisMaxChunk
+  int64_t block;               // fresh vertices per round, a multiple of 512
+  int64_t region;              // entries per list region: ceil(n / kMisStripes), a list chunk
+                               // and a set of fresh vertices
   int32_t sorted;              // rows ascending: the lower neighbours are a prefix
   int32_t pad;
 };

@@ -141,15 +141,6 @@ __device__ __forceinline__ int wave_max(int x) {
   return x;
 }
 
-// Orders this wavefront's LDS writes before its later LDS reads by other
-// lanes.  The fences name LDS only: a fence on all memory would also wait for
-// every global store in flight (loads and stores share one counter here).
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-}
-
 __device__ __forceinline__ uint32_t shfl_off(uint32_t x, int src) { return __shfl(x, src); }
 __device__ __forceinline__ int64_t shfl_off(int64_t x, int src) {
   return (int64_t)__shfl((long long)x, src);

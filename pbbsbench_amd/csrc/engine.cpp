@@ -65,8 +65,12 @@ hipError_t launch_mis_init(const MisArgs<OffT>& a, int grid, hipStream_t stream)
 template <typename OffT>
 hipError_t launch_mis_round(const MisArgs<OffT>& a, int step, int grid, hipStream_t stream);
 template <typename OffT>
-hipError_t launch_mis_output(const MisArgs<OffT>& a, int32_t* flags_out,
-                             unsigned long long* members, int grid, hipStream_t stream);
+hipError_t launch_mis_small(const MisArgs<OffT>& a, int32_t* flags_out, hipStream_t stream);
+template <typename OffT>
+const void* mis_round_symbol(int step);
+template <typename OffT>
+hipError_t launch_mis_output(const MisArgs<OffT>& a, int32_t* flags_out, int grid,
+                             hipStream_t stream);
 hipError_t launch_st_init(const StArgs& a, int grid, hipStream_t stream);
 hipError_t launch_st_round(const StArgs& a, long long round, int grid, hipStream_t stream);
 hipError_t launch_st_tree(const StArgs& a, long long round, int grid, hipStream_t stream);
@@ -222,12 +226,12 @@ struct pbbs_ctx {
   uint32_t* m_wg = nullptr;              // [kMaxMultiJobs + 1]
   int32_t* m_host_status = nullptr;      // pinned: 16 words per job
   BfsState* m_host_state = nullptr;      // pinned: one per job
-  // maximal independent set: per-vertex flags and row positions, the two
+  // maximal independent set: per-vertex states and row positions, the two
   // worklists (kMisStripes regions each), the int32 output staged for a host
-  // copy, the control words (three sets of region counts, the finished flag,
-  // the set's size), per-workgroup member counts and round counters
+  // copy, the control words (three sets of region counts, the finished flag),
+  // per-workgroup member counts and round counters
   int64_t cap_sn = 0;
-  uint8_t* s_flags = nullptr;
+  unsigned long long* s_state = nullptr;
   uint32_t* s_pos = nullptr;
   int32_t* s_list = nullptr;             // list0 | list1, kMisStripes * mis_region(cap_sn) each
   int32_t* s_out = nullptr;
@@ -321,12 +325,13 @@ static void free_workspace(pbbs_ctx* c) {
 }
 
 // Control words of a set run: three sets of kMisStripes region counts, one
-// per 128-byte line, then the finished flag and the set's size.
+// per 128-byte line, then the finished flag.
 constexpr int kMisCtlFinished = 3 * kMisStripes * 16;
-constexpr int kMisCtlMembers = kMisCtlFinished + 8;
-constexpr int kMisCtlWords = kMisCtlMembers + 8;
+constexpr int kMisCtlWords = kMisCtlFinished + 8;
 
-static int64_t mis_region(int64_t n) { return (n + kMisStripes - 1) / kMisStripes + kMisMaxChunk; }
+static int64_t mis_region(int64_t n) {
+  return (n + kMisStripes - 1) / kMisStripes + kMisMaxChunk + kMisPer * kWave + 2;
+}
 
 constexpr int kStCounts = kStMaxGroups + 2 * kStMaxTiles;
 
@@ -375,7 +380,7 @@ static int ensure_st_workspace(pbbs_ctx* c, int64_t n, int64_t r, int64_t e) {
 }
 
 static void free_mis_workspace(pbbs_ctx* c) {
-  (void)hipFree(c->s_flags);
+  (void)hipFree(c->s_state);
   (void)hipFree(c->s_pos);
   (void)hipFree(c->s_list);
   (void)hipFree(c->s_out);
@@ -383,7 +388,7 @@ static void free_mis_workspace(pbbs_ctx* c) {
   (void)hipFree(c->s_part);
   (void)hipFree(c->s_wg);
   c->s_part = nullptr;
-  c->s_flags = nullptr;
+  c->s_state = nullptr;
   c->s_pos = nullptr;
   c->s_list = c->s_out = nullptr;
   c->s_ctl = nullptr;
@@ -394,7 +399,7 @@ static void free_mis_workspace(pbbs_ctx* c) {
 static int ensure_mis_workspace(pbbs_ctx* c, int64_t n) {
   if (n <= c->cap_sn) return PBBS_OK;
   free_mis_workspace(c);
-  if (hipMalloc(&c->s_flags, n) != hipSuccess ||
+  if (hipMalloc(&c->s_state, mis_state_words(n) * sizeof(unsigned long long)) != hipSuccess ||
       hipMalloc(&c->s_pos, n * sizeof(uint32_t)) != hipSuccess ||
       hipMalloc(&c->s_list, 2 * kMisStripes * mis_region(n) * sizeof(int32_t)) != hipSuccess ||
       hipMalloc(&c->s_out, n * sizeof(int32_t)) != hipSuccess ||
@@ -699,13 +704,13 @@ int pbbs_graph_upload(pbbs_ctx* c, int64_t n, int64_t m, const void* offsets, co
   const hipMemcpyKind kind =
       (flags & PBBS_GRAPH_DEVICE_INPUT) ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
   if (hipMalloc(&g->d_off, (n + 1) * osz) != hipSuccess ||
-      hipMalloc(&g->d_adj, std::max<int64_t>(m, 1) * sizeof(int32_t)) != hipSuccess ||
+      hipMalloc(&g->d_adj, (m + kAdjPad) * sizeof(int32_t)) != hipSuccess ||
       hipMalloc(&g->d_iso, nwords * sizeof(unsigned long long)) != hipSuccess) {
     pbbs_graph_free(g);
     return fail(PBBS_ERR_NOMEM, "graph allocation (n=%lld, m=%lld) failed", (long long)n,
                 (long long)m);
   }
-  g->device_bytes = (n + 1) * osz + std::max<int64_t>(m, 1) * 4 + nwords * 8;
+  g->device_bytes = (n + 1) * osz + (m + kAdjPad) * 4 + nwords * 8;
   if (hipMemcpyAsync(g->d_off, offsets, (n + 1) * osz, kind, c->stream) != hipSuccess ||
       (m > 0 && hipMemcpyAsync(g->d_adj, adj, m * sizeof(int32_t), kind, c->stream) != hipSuccess) ||
       hipStreamSynchronize(c->stream) != hipSuccess) {
@@ -1335,18 +1340,21 @@ extern "C" int pbbs_bfs(pbbs_ctx* c, pbbs_graph* g, int32_t source, int32_t* par
 }
 
 // ------------------------------------------------- maximal independent set
-// Rounds run in chunks of 8 launches on the context's stream (the
-// relabelled benchmark graphs finish in 6-9 rounds, and a launch after the
-// last round still costs its dispatch); after each chunk the host reads whether a round found the worklist
-// empty.  A round decides at least the lowest undecided vertex (its lower
-// neighbours were all decided before the round began), so n + 1 rounds end
-// any run; more means a fault, reported as an error.
+// The first chunk covers the blocks of fresh vertices and kMisTail rounds more
+// (the relabelled benchmark graphs need 3 after their last block), with the
+// output launched behind it, so that most runs meet the host once; a run that
+// is not over by then goes on in chunks of 8, and writes its output again.  A
+// round decides at least the lowest undecided vertex (its lower neighbours
+// were all decided before the round began), so n + 1 rounds past the blocks
+// end any run; more means a fault, reported as an error.
+constexpr int kMisTail = 4;
+
 template <typename OffT>
 static int run_mis(pbbs_ctx* c, pbbs_graph* g, int32_t* d_out, pbbs_mis_stats* stats) {
   MisArgs<OffT> a{};
   a.off = static_cast<const OffT*>(g->d_off);
   a.adj = g->d_adj;
-  a.flags = c->s_flags;
+  a.state = c->s_state;
   a.pos = c->s_pos;
   a.region = mis_region(c->cap_sn);
   a.list[0] = c->s_list;
@@ -1358,21 +1366,45 @@ static int run_mis(pbbs_ctx* c, pbbs_graph* g, int32_t* d_out, pbbs_mis_stats* s
   a.host_status = c->host_status;
   a.n = g->n;
   a.sorted = g->sorted ? 1 : 0;
-  const int64_t need = (g->n + kBlock - 1) / kBlock;
-  const int grid = (int)std::min<int64_t>(std::max<int64_t>(need, 1), 8 * c->num_cus);
+  const int64_t need = std::max<int64_t>((g->n + kBlock - 1) / kBlock, 1);
+  const int pass_grid = (int)std::min<int64_t>(need, 8 * c->num_cus);   // init and output
   // row entries per look: 4 where rows average 16 entries or more, else 2
   // (measured on the benchmark's rMat, randLocal and 3D-grid graphs)
   const int step = g->m >= 16 * g->n ? 4 : 2;
+  // the workgroups resident at once: they share a block's sets evenly
+  int per_cu = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, mis_round_symbol<OffT>(step), kBlock,
+                                                   0) != hipSuccess ||
+      per_cu < 1)
+    per_cu = 1;
+  const int grid = (int)std::min<int64_t>(need, (int64_t)per_cu * c->num_cus);
+  // Fresh vertices per round: two sets per resident wavefront, or n / 16 where
+  // that is more, but two blocks at least: a smaller block meets fewer
+  // undecided neighbours, and a round costs 4-8 us however small (2^18 to 2^21
+  // vertices: 1, 2, 4 and 8 blocks at least measured 223/275/322, 174/210/251,
+  // 184/212/257 and 221/246/281 us).
+  const int64_t two_sets = (int64_t)grid * kWavesPerBlock * 2 * kMisPer * kWave;
+  a.block = std::min(std::max<int64_t>(two_sets, g->n / 16), (g->n + 1) / 2);
+  a.block = (a.block + 511) / 512 * 512;
+  int blocks = 0;
+  while (mis_block_start(a.block, g->n, blocks) < g->n) ++blocks;
   volatile int32_t* hs = c->host_status;
   HIP_TRY(hipEventRecord(c->ev_start, c->stream));
-  HIP_TRY(launch_mis_init<OffT>(a, grid, c->stream));
-  const int64_t limit = g->n + 2;
+  const bool small = g->n <= kMisSmall;
+  if (small) {
+    HIP_TRY(launch_mis_small<OffT>(a, d_out, c->stream));
+    HIP_TRY(hipEventRecord(c->ev_end, c->stream));
+    HIP_TRY(hipEventSynchronize(c->ev_end));
+  } else {
+    HIP_TRY(launch_mis_init<OffT>(a, pass_grid, c->stream));
+  }
+  const int64_t limit = g->n + 2 + blocks;
   int64_t launched = 0;
-  const int K = 8;
-  for (;;) {
+  for (int64_t K = blocks + kMisTail; !small; K = 8) {
     const int k = (int)std::min<int64_t>(K, limit - launched);
     for (int i = 0; i < k; ++i) HIP_TRY(launch_mis_round<OffT>(a, step, grid, c->stream));
     launched += k;
+    HIP_TRY(launch_mis_output<OffT>(a, d_out, pass_grid, c->stream));
     HIP_TRY(hipEventRecord(c->ev_end, c->stream));
     HIP_TRY(hipEventSynchronize(c->ev_end));
     if (hs[2]) return fail(PBBS_ERR_STATE, "set worklist region overflow");
@@ -1381,18 +1413,12 @@ static int run_mis(pbbs_ctx* c, pbbs_graph* g, int32_t* d_out, pbbs_mis_stats* s
       return fail(PBBS_ERR_STATE, "set rounds did not finish in %lld launches",
                   (long long)launched);
   }
-  const int32_t rounds = hs[1];
-  HIP_TRY(launch_mis_output<OffT>(a, d_out, c->s_ctl + kMisCtlMembers, grid, c->stream));
-  HIP_TRY(hipMemcpyAsync(c->host_status + 4, c->s_ctl + kMisCtlMembers, sizeof(unsigned long long),
-                         hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipEventRecord(c->ev_end, c->stream));
-  HIP_TRY(hipEventSynchronize(c->ev_end));
   if (stats) {
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, c->ev_start, c->ev_end));
     unsigned long long members = 0;
     std::memcpy(&members, c->host_status + 4, sizeof(members));
-    stats->rounds = rounds;
+    stats->rounds = hs[1];
     stats->pad = 0;
     stats->members = (int64_t)members;
     stats->device_ms = ms;
@@ -2046,8 +2072,8 @@ int64_t ctx_workspace_bytes(const pbbs_ctx* c) {
   if (c->t_ctl)
     b += 12 * c->cap_tn + (c->cap_tn + 63) / 64 * 8 + 16 * c->cap_tr + 8 * c->cap_te +
          kStCounts * 4;
-  if (c->s_flags)
-    b += 9 * c->cap_sn + 8 * kMisStripes * mis_region(c->cap_sn) + kMisCtlWords * 8 +
+  if (c->s_state)
+    b += mis_state_words(c->cap_sn) * 8 + 8 * c->cap_sn + 8 * kMisStripes * mis_region(c->cap_sn) + kMisCtlWords * 8 +
          kMaxGrid * 12;
   return b;
 }

@@ -1,4 +1,4 @@
-// Typed global-memory pointers for the HIP kernels.
+// Memory helpers of the HIP kernels: typed global pointers, wavefront LDS order.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -20,6 +20,15 @@ __device__ __forceinline__ gptr<T> glob(T* p) {
 template <typename T>
 __device__ __forceinline__ T* gen(gptr<T> p) {
   return (T*)p;
+}
+
+// Orders this wavefront's LDS writes before its later LDS reads by other
+// lanes.  The fences name LDS only: a fence on all memory would also wait for
+// every global store in flight (loads and stores share one counter here).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 }
 
 }  // namespace pbbs
