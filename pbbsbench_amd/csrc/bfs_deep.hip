@@ -39,7 +39,7 @@
 #include <stdint.h>
 
 #include "bfs_device.hpp"
-#include "gmem.hpp"
+#include "device_util.hpp"
 
 namespace pbbs {
 

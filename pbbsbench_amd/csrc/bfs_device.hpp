@@ -118,6 +118,22 @@ struct BfsArgs {
 // workgroup of each (njobs + 1 entries, the last one the grid size).
 constexpr int kMaxMultiJobs = 64;
 
+// -------------------------------------------------------- small graphs
+// A whole BFS in one workgroup (bfs_small.hip).
+constexpr int kSmallBlock = 1024;
+constexpr int kSmallMaxN = 16384;    // vertices its LDS holds (8 bytes each)
+
+struct BfsSmallJob {
+  const void* off;        // offsets[n+1], of the launch's width
+  const int32_t* adj;
+  int32_t* parent;        // out, device or pinned host memory, or null
+  int32_t* depth;
+  int32_t* host_status;   // pinned: [0] done, [1] levels
+  BfsState* host_state;   // pinned: the totals
+  int32_t n;
+  int32_t source;
+};
+
 // --------------------------------------------------------- deep graphs
 // A persistent launch that meets every few levels (bfs_deep.hip).
 constexpr int kDeepBlock = 256;        // threads per workgroup

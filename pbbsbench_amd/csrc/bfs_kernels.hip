@@ -33,7 +33,7 @@
 #include <rocprim/iterator/counting_iterator.hpp>
 
 #include "bfs_device.hpp"
-#include "gmem.hpp"
+#include "device_util.hpp"
 
 namespace pbbs {
 
@@ -45,20 +45,6 @@ __device__ __forceinline__ unsigned lanes_below(unsigned long long mask) {
   return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
                                    __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
 }
-
-// Cross-lane moves through DPP (a VALU operand modifier, a few cycles)
-// instead of ds_bpermute (an LDS round trip).  `old` is what lanes without a
-// source lane (or masked rows) receive.
-template <int kCtrl, int kRowMask>
-__device__ __forceinline__ unsigned dpp_u32(unsigned x, unsigned old) {
-  return (unsigned)__builtin_amdgcn_update_dpp((int)old, (int)x, kCtrl, kRowMask, 0xf, false);
-}
-template <int kCtrl, int kRowMask>
-__device__ __forceinline__ int dpp_i32(int x, int old) {
-  return __builtin_amdgcn_update_dpp(old, x, kCtrl, kRowMask, 0xf, false);
-}
-constexpr int kRowShr1 = 0x111, kRowShr2 = 0x112, kRowShr4 = 0x114, kRowShr8 = 0x118;
-constexpr int kRowBcast15 = 0x142, kRowBcast31 = 0x143, kWaveShr1 = 0x138;
 
 // One step of a keyed (segmented) inclusive OR scan: lanes take the value
 // of the source lane when it carries the same key.  Keys are non-decreasing
@@ -118,17 +104,6 @@ __device__ __forceinline__ unsigned long long seg_or_scan_d(unsigned long long x
   PBBS_SEG_STEP(kRowBcast31, 0xc, false, dist > lane32)
 #undef PBBS_SEG_STEP
   return ((unsigned long long)hi << 32) | lo;
-}
-
-// Inclusive sum over the wavefront through DPP.
-__device__ __forceinline__ unsigned wave_inclusive_sum_dpp(unsigned x) {
-  x += dpp_u32<kRowShr1, 0xf>(x, 0u);
-  x += dpp_u32<kRowShr2, 0xf>(x, 0u);
-  x += dpp_u32<kRowShr4, 0xf>(x, 0u);
-  x += dpp_u32<kRowShr8, 0xf>(x, 0u);
-  x += dpp_u32<kRowBcast15, 0xa>(x, 0u);
-  x += dpp_u32<kRowBcast31, 0xc>(x, 0u);
-  return x;
 }
 
 __device__ __forceinline__ unsigned wave_inclusive_sum(unsigned x) {

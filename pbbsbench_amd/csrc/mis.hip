@@ -29,7 +29,7 @@
 #include <climits>
 
 #include "bfs_device.hpp"
-#include "gmem.hpp"
+#include "device_util.hpp"
 
 namespace pbbs {
 
