@@ -1299,12 +1299,13 @@ __global__ __launch_bounds__(kBlock) void bfs_multi_kernel(
   if (threadIdx.x == 0) A->wg_level[vb] = (uint32_t)k;
 }
 
+// Presets one BFS from s: outputs, bitmaps, level counters, F_0 = {s} and the
+// control block, as thread tid of nth; thread 0 writes the argument block to
+// *dst unless it is there already (dst null).
 template <typename OffT>
-__global__ __launch_bounds__(kBlock) void bfs_init_kernel(BfsArgs<OffT> a, BfsArgs<OffT>* dst,
-                                                          const unsigned long long* __restrict__ iso,
-                                                          int32_t s) {
-  const long long tid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long nth = (long long)gridDim.x * blockDim.x;
+__device__ __forceinline__ void bfs_preset(const BfsArgs<OffT>& a, BfsArgs<OffT>* dst,
+                                           const unsigned long long* __restrict__ iso, int32_t s,
+                                           long long tid, long long nth) {
   const int32_t n = (int32_t)a.n;
   for (long long i = tid; i < a.n; i += nth) {
     a.parent[i] = (i == s) ? s : -1;
@@ -1326,9 +1327,11 @@ __global__ __launch_bounds__(kBlock) void bfs_init_kernel(BfsArgs<OffT> a, BfsAr
   if (a.deep_words)
     for (long long i = tid; i < 2 * kDeepMaxGroups; i += nth) a.deep_words[i] = 0;
   if (tid == 0) {
-    BfsArgs<OffT> b = a;
-    b.iso = iso;
-    *dst = b;
+    if (dst) {
+      BfsArgs<OffT> b = a;
+      b.iso = iso;
+      *dst = b;
+    }
     const unsigned long long deg = (unsigned long long)(a.off[s + 1] - a.off[s]);
     BfsState* st = a.st;
     a.q[0][0] = s;
@@ -1356,6 +1359,24 @@ __global__ __launch_bounds__(kBlock) void bfs_init_kernel(BfsArgs<OffT> a, BfsAr
     __hip_atomic_store(&a.host_status[1], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __hip_atomic_store(&a.host_status[0], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
+}
+
+template <typename OffT>
+__global__ __launch_bounds__(kBlock) void bfs_init_kernel(BfsArgs<OffT> a, BfsArgs<OffT>* dst,
+                                                          const unsigned long long* __restrict__ iso,
+                                                          int32_t s) {
+  bfs_preset(a, dst, iso, s, (long long)blockIdx.x * blockDim.x + threadIdx.x,
+             (long long)gridDim.x * blockDim.x);
+}
+
+// The presets of a multi-graph launch's jobs, blockIdx.y's by blockIdx.x (one
+// launch for all of them: one each took 4 us a job).
+template <typename OffT>
+__global__ __launch_bounds__(kBlock) void bfs_multi_init_kernel(
+    const BfsArgs<OffT>* __restrict__ args, const int32_t* __restrict__ sources) {
+  const BfsArgs<OffT> a = args[blockIdx.y];
+  bfs_preset(a, static_cast<BfsArgs<OffT>*>(nullptr), a.iso, sources[blockIdx.y],
+             (long long)blockIdx.x * blockDim.x + threadIdx.x, (long long)gridDim.x * blockDim.x);
 }
 
 // ---------------------------------------------------------------- batched BFS
@@ -2547,8 +2568,13 @@ const void* multi_kernel_symbol(bool sorted) {
 }
 
 template <typename OffT>
-hipError_t launch_bfs_multi(const BfsArgs<OffT>* args, const uint32_t* wg_begin, int njobs,
-                            bool sorted, int grid, hipStream_t stream) {
+hipError_t launch_bfs_multi(const BfsArgs<OffT>* args, const uint32_t* wg_begin,
+                            const int32_t* sources, int njobs, bool sorted, int init_grid,
+                            int grid, hipStream_t stream) {
+  hipLaunchKernelGGL(bfs_multi_init_kernel<OffT>, dim3(init_grid, njobs), dim3(kBlock), 0, stream,
+                     args, sources);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || grid == 0) return e;   // the presets alone
   if (sorted)
     hipLaunchKernelGGL((bfs_multi_kernel<OffT, true>), dim3(grid), dim3(kBlock), 0, stream, args,
                        wg_begin, njobs);
@@ -2763,8 +2789,8 @@ hipError_t launch_mbfs_depth(const MbfsArgs<OffT>& a, int grid, hipStream_t stre
   template hipError_t launch_bfs_level<OffT>(const BfsArgs<OffT>*, int, int, hipStream_t);       \
   template const void* persist_kernel_symbol<OffT>(int);                                        \
   template const void* multi_kernel_symbol<OffT>(bool);                                         \
-  template hipError_t launch_bfs_multi<OffT>(const BfsArgs<OffT>*, const uint32_t*, int, bool,   \
-                                            int, hipStream_t);                                   \
+  template hipError_t launch_bfs_multi<OffT>(const BfsArgs<OffT>*, const uint32_t*,              \
+                                            const int32_t*, int, bool, int, int, hipStream_t);   \
   template hipError_t launch_bfs_persist<OffT>(const BfsArgs<OffT>*, int, int, hipStream_t);     \
   template hipError_t launch_graph_offsets<OffT>(const OffT*, long long, long long,             \
                                                  unsigned long long*, unsigned long long*, int,  \

@@ -7,6 +7,7 @@
 #include <atomic>
 #include <chrono>
 #include <cstdarg>
+#include <cstddef>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -35,8 +36,9 @@ const void* persist_kernel_symbol(int variant);
 template <typename OffT>
 const void* multi_kernel_symbol(bool sorted);
 template <typename OffT>
-hipError_t launch_bfs_multi(const BfsArgs<OffT>* args, const uint32_t* wg_begin, int njobs,
-                            bool sorted, int grid, hipStream_t stream);
+hipError_t launch_bfs_multi(const BfsArgs<OffT>* args, const uint32_t* wg_begin,
+                            const int32_t* sources, int njobs, bool sorted, int init_grid,
+                            int grid, hipStream_t stream);
 template <typename OffT>
 hipError_t launch_bfs_small(const BfsSmallJob* jobs, int njobs, const BfsSmallJob& one,
                             hipStream_t stream);
@@ -147,6 +149,16 @@ struct SingleWs {
   void* args = nullptr;
 };
 
+// What one launch of a multi-graph call reads: argument blocks of either
+// offset width, first workgroups and sources, or the jobs of a small launch.
+struct MultiParams {
+  alignas(16) unsigned char args[kMaxMultiJobs * sizeof(BfsArgs<int64_t>)];
+  uint32_t wg[kMaxMultiJobs + 1];
+  int32_t sources[kMaxMultiJobs];
+  BfsSmallJob small[kMaxMultiJobs];
+};
+constexpr int kMultiLaunches = 6;   // small jobs by width, others by width and row order
+
 struct pbbs_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -224,12 +236,16 @@ struct pbbs_ctx {
   // pinned memory that host outputs pass through
   int32_t* p_out = nullptr;
   int64_t cap_pout = 0;                  // entries
-  // multi-graph launches: the jobs' workspaces, their argument blocks and
-  // first workgroups, and pinned status words and control-block copies
+  // multi-graph launches: the jobs' workspaces, their outputs (the parents of
+  // all jobs, then the depths), a parameter block for every launch (device,
+  // and pinned to upload from), and pinned status words and control-block
+  // copies
   unsigned char* m_ws = nullptr;
   int64_t m_ws_bytes = 0;
-  void* m_args = nullptr;                // BfsArgs<int64_t>[kMaxMultiJobs]
-  uint32_t* m_wg = nullptr;              // [kMaxMultiJobs + 1]
+  int32_t* m_out = nullptr;
+  int64_t cap_mout = 0;                  // entries
+  MultiParams* m_params = nullptr;       // [kMultiLaunches]
+  MultiParams* m_host_params = nullptr;
   int32_t* m_host_status = nullptr;      // pinned: 16 words per job
   BfsState* m_host_state = nullptr;      // pinned: one per job
   // maximal independent set: per-vertex states and row positions, the two
@@ -542,8 +558,9 @@ int pbbs_ctx_destroy(pbbs_ctx* c) {
   (void)hipFree(c->w_wg_level);
   (void)hipFree(c->w_args);
   (void)hipFree(c->m_ws);
-  (void)hipFree(c->m_args);
-  (void)hipFree(c->m_wg);
+  (void)hipFree(c->m_out);
+  (void)hipFree(c->m_params);
+  if (c->m_host_params) (void)hipHostFree(c->m_host_params);
   if (c->p_out) (void)hipHostFree(c->p_out);
   if (c->m_host_status) (void)hipHostFree(c->m_host_status);
   if (c->m_host_state) (void)hipHostFree(c->m_host_state);
@@ -2344,14 +2361,9 @@ static BfsArgs<OffT> job_args(pbbs_ctx* c, pbbs_graph* g, const JobLayout& L, un
   return a;
 }
 
-int64_t multi_workspace_bytes(const int64_t* n, int32_t njobs, int32_t queue_div) {
-  int64_t b = 0;
-  for (int32_t j = 0; j < njobs; ++j) b += job_layout(n[j], queue_div, true).total;
-  return b;
-}
-
 // Workgroups per job: proportional to n + m (at least one each, at most one
-// per 4096 edges, so a small graph does not spread over the whole device),
+// per 65536 edges: 16 graphs of scales 10-17 take 476 us a call with one per
+// 4096, 410 with one per 32768 to 65536, 516 with one per 131072),
 // within cap in total.
 static void split_grid(const std::vector<pbbs_graph*>& gs, int cap, std::vector<uint32_t>& wg) {
   const size_t J = gs.size();
@@ -2361,7 +2373,7 @@ static void split_grid(const std::vector<pbbs_graph*>& gs, int cap, std::vector<
   int64_t sum = 0;
   for (size_t j = 0; j < J; ++j) {
     const int64_t share = (int64_t)((double)cap * (double)(gs[j]->n + gs[j]->m) / total);
-    const int64_t most = std::max<int64_t>(1, (gs[j]->m + 4095) / 4096);
+    const int64_t most = std::max<int64_t>(1, (gs[j]->m + 65535) / 65536);
     w[j] = std::max<int64_t>(1, std::min(share, most));
     sum += w[j];
   }
@@ -2376,12 +2388,50 @@ static void split_grid(const std::vector<pbbs_graph*>& gs, int cap, std::vector<
   for (size_t j = 0; j < J; ++j) wg[j + 1] = wg[j] + (uint32_t)w[j];
 }
 
+// The stats of a job that a shared launch finished.
+static void shared_stats(const BfsState& h, float ms, pbbs_bfs_stats& st) {
+  std::memset(&st, 0, sizeof st);
+  st.levels = h.max_depth + 1;
+  st.td_levels = h.td_levels;
+  st.bu_levels = h.bu_levels;
+  st.launches = 1;
+  st.reached = (int64_t)h.reached;
+  st.edges_reached = (int64_t)h.edges_reached;
+  st.device_ms = ms;
+}
+
+// One launch of small jobs, a workgroup each.
+static int run_multi_small(pbbs_ctx* c, MultiParams* host, MultiParams* dev,
+                           const std::vector<int>& ids, const std::vector<pbbs_graph*>& graphs,
+                           const int32_t* sources, const std::vector<int32_t*>& dpar,
+                           const std::vector<int32_t*>& ddep, pbbs_bfs_stats* stats, bool off64) {
+  const int J = (int)ids.size();
+  for (int j = 0; j < J; ++j)
+    host->small[j] = small_job(graphs[ids[j]], sources[ids[j]], dpar[ids[j]], ddep[ids[j]],
+                               c->m_host_status + 16 * j, c->m_host_state + j);
+  HIP_TRY(hipMemcpyAsync(dev->small, host->small, J * sizeof(BfsSmallJob), hipMemcpyHostToDevice,
+                         c->stream));
+  HIP_TRY(hipEventRecord(c->ev_start, c->stream));
+  HIP_TRY(off64 ? launch_bfs_small<int64_t>(dev->small, J, BfsSmallJob{}, c->stream)
+                : launch_bfs_small<uint32_t>(dev->small, J, BfsSmallJob{}, c->stream));
+  HIP_TRY(hipEventRecord(c->ev_end, c->stream));
+  HIP_TRY(hipEventSynchronize(c->ev_end));
+  float ms = 0.f;
+  HIP_TRY(hipEventElapsedTime(&ms, c->ev_start, c->ev_end));
+  for (int j = 0; j < J; ++j) {
+    if (!c->m_host_status[16 * j])
+      return fail(PBBS_ERR_STATE, "small-graph launch did not finish");
+    shared_stats(c->m_host_state[j], ms, stats[ids[j]]);
+  }
+  return PBBS_OK;
+}
+
 template <typename OffT>
-static int run_multi_group(pbbs_ctx* c, const std::vector<int>& ids,
-                           const std::vector<pbbs_graph*>& graphs, const int32_t* sources,
-                           const std::vector<JobLayout>& L, const std::vector<int64_t>& at,
-                           std::vector<int32_t*>& dpar, std::vector<int32_t*>& ddep,
-                           pbbs_bfs_stats* stats, bool sorted) {
+static int run_multi_group(pbbs_ctx* c, MultiParams* host, MultiParams* dev,
+                           const std::vector<int>& ids, const std::vector<pbbs_graph*>& graphs,
+                           const int32_t* sources, const std::vector<JobLayout>& L,
+                           const std::vector<int64_t>& at, const std::vector<int32_t*>& dpar,
+                           const std::vector<int32_t*>& ddep, pbbs_bfs_stats* stats, bool sorted) {
   const int J = (int)ids.size();
   std::vector<pbbs_graph*> gs(J);
   for (int j = 0; j < J; ++j) gs[j] = graphs[ids[j]];
@@ -2394,24 +2444,32 @@ static int run_multi_group(pbbs_ctx* c, const std::vector<int>& ids,
   if (J > cap) return fail(PBBS_ERR_LIMIT, "%d jobs exceed the %d workgroups resident", J, cap);
   std::vector<uint32_t> wg;
   split_grid(gs, cap, wg);
-  BfsArgs<OffT>* dargs = static_cast<BfsArgs<OffT>*>(c->m_args);
+  BfsArgs<OffT>* hargs = reinterpret_cast<BfsArgs<OffT>*>(host->args);
+  BfsArgs<OffT>* dargs = reinterpret_cast<BfsArgs<OffT>*>(dev->args);
+  int64_t most = 1;
   for (int j = 0; j < J; ++j) {
     const int i = ids[j];
-    unsigned char* base = c->m_ws + at[i];
     int32_t* hs = c->m_host_status + 16 * j;
     hs[0] = hs[1] = hs[2] = 0;
-    const BfsArgs<OffT> a =
-        job_args<OffT>(c, gs[j], L[i], base, dpar[i], ddep[i], hs, c->m_host_state + j);
-    const int init_grid = (int)std::max<int64_t>(
-        1, std::min<int64_t>((gs[j]->n + kBlock - 1) / kBlock, c->num_cus * 16));
-    HIP_TRY(launch_bfs_init<OffT>(a, dargs + j, gs[j]->d_iso, sources[i], init_grid, c->stream));
+    hargs[j] = job_args<OffT>(c, gs[j], L[i], c->m_ws + at[i], dpar[i], ddep[i], hs,
+                              c->m_host_state + j);
+    hargs[j].iso = gs[j]->d_iso;
+    host->wg[j] = wg[j];
+    host->sources[j] = sources[i];
+    most = std::max(most, gs[j]->n);
   }
-  HIP_TRY(hipMemcpyAsync(c->m_wg, wg.data(), (J + 1) * sizeof(uint32_t), hipMemcpyHostToDevice,
+  host->wg[J] = wg[J];
+  HIP_TRY(hipMemcpyAsync(dev, host, offsetof(MultiParams, small), hipMemcpyHostToDevice,
                          c->stream));
+  const int init_grid =
+      (int)std::min<int64_t>((most + kBlock - 1) / kBlock, std::max(1, c->num_cus * 16 / J));
   const bool persist = take_persist(c);
   if (persist) {
-    HIP_TRY(hipEventRecord(c->ev_start, c->stream));
-    const hipError_t le = launch_bfs_multi<OffT>(dargs, c->m_wg, J, sorted, (int)wg[J], c->stream);
+    const hipError_t be = hipEventRecord(c->ev_start, c->stream);
+    const hipError_t le =
+        be == hipSuccess ? launch_bfs_multi<OffT>(dargs, dev->wg, dev->sources, J, sorted,
+                                                  init_grid, (int)wg[J], c->stream)
+                         : be;
     const hipError_t re = le == hipSuccess ? hipEventRecord(c->ev_end, c->stream) : le;
     const hipError_t se = re == hipSuccess ? hipEventSynchronize(c->ev_end) : re;
     release_persist(c);
@@ -2424,16 +2482,7 @@ static int run_multi_group(pbbs_ctx* c, const std::vector<int>& ids,
     const int i = ids[j];
     volatile int32_t* hs = c->m_host_status + 16 * j;
     if (persist && hs[0]) {
-      const BfsState& h = c->m_host_state[j];
-      pbbs_bfs_stats& st = stats[i];
-      std::memset(&st, 0, sizeof st);
-      st.levels = h.max_depth + 1;
-      st.td_levels = h.td_levels;
-      st.bu_levels = h.bu_levels;
-      st.launches = 1;
-      st.reached = (int64_t)h.reached;
-      st.edges_reached = (int64_t)h.edges_reached;
-      st.device_ms = ms;
+      shared_stats(c->m_host_state[j], ms, stats[i]);
       continue;
     }
     // the device was busy with another persistent launch, or this job's
@@ -2451,6 +2500,32 @@ static int run_multi_group(pbbs_ctx* c, const std::vector<int>& ids,
 // Jobs on graphs with more edges than this run alone inside pbbs_bfs_multi.
 constexpr int64_t kMultiAloneEdges = int64_t(1) << 23;
 
+// The buffers of multi-graph calls that do not depend on the jobs.
+static int ensure_multi(pbbs_ctx* c) {
+  if (c->m_params) return PBBS_OK;
+  MultiParams *dev = nullptr, *host = nullptr;
+  int32_t* hs = nullptr;
+  BfsState* hst = nullptr;
+  if (hipMalloc(&dev, kMultiLaunches * sizeof(MultiParams)) != hipSuccess ||
+      hipHostMalloc((void**)&host, kMultiLaunches * sizeof(MultiParams), hipHostMallocDefault) !=
+          hipSuccess ||
+      hipHostMalloc((void**)&hs, kMaxMultiJobs * 16 * sizeof(int32_t), hipHostMallocCoherent) !=
+          hipSuccess ||
+      hipHostMalloc((void**)&hst, kMaxMultiJobs * sizeof(BfsState), hipHostMallocDefault) !=
+          hipSuccess) {
+    (void)hipGetLastError();
+    (void)hipFree(dev);
+    if (host) (void)hipHostFree(host);
+    if (hs) (void)hipHostFree(hs);
+    return fail(PBBS_ERR_NOMEM, "multi-graph control buffers failed");
+  }
+  c->m_host_params = host;
+  c->m_host_status = hs;
+  c->m_host_state = hst;
+  c->m_params = dev;
+  return PBBS_OK;
+}
+
 extern "C" int pbbs_bfs_multi(pbbs_ctx* c, int32_t njobs, pbbs_graph* const* graphs,
                               const int32_t* sources, int32_t* const* parents,
                               int32_t* const* depths, uint32_t out_flags, pbbs_bfs_stats* stats) {
@@ -2467,44 +2542,25 @@ extern "C" int pbbs_bfs_multi(pbbs_ctx* c, int32_t njobs, pbbs_graph* const* gra
                   (long long)g->n);
   }
   HIP_TRY(hipSetDevice(c->device));
-  if (!c->m_args) {
-    void* args = nullptr;
-    uint32_t* wg = nullptr;
-    int32_t* hs = nullptr;
-    BfsState* hst = nullptr;
-    if (hipMalloc(&args, kMaxMultiJobs * sizeof(BfsArgs<int64_t>)) != hipSuccess ||
-        hipMalloc(&wg, (kMaxMultiJobs + 1) * sizeof(uint32_t)) != hipSuccess ||
-        hipHostMalloc((void**)&hs, kMaxMultiJobs * 16 * sizeof(int32_t), hipHostMallocCoherent) !=
-            hipSuccess ||
-        hipHostMalloc((void**)&hst, kMaxMultiJobs * sizeof(BfsState), hipHostMallocDefault) !=
-            hipSuccess) {
-      (void)hipGetLastError();
-      (void)hipFree(args);
-      (void)hipFree(wg);
-      if (hs) (void)hipHostFree(hs);
-      if (hst) (void)hipHostFree(hst);
-      return fail(PBBS_ERR_NOMEM, "multi-graph control buffers failed");
-    }
-    c->m_wg = wg;
-    c->m_host_status = hs;
-    c->m_host_state = hst;
-    c->m_args = args;
-  }
+  int rc = ensure_multi(c);
+  if (rc != PBBS_OK) return rc;
   // as in pbbs_bfs_batch: deterministic outputs meet the any-parent contract
   if (out_flags & ~(PBBS_OUT_DEVICE | PBBS_BFS_ANY_PARENT))
     return fail(PBBS_ERR_INVALID, "unknown flags 0x%x", out_flags);
   const bool dev_out = (out_flags & PBBS_OUT_DEVICE) != 0;
   std::vector<pbbs_graph*> gs(graphs, graphs + njobs);
-  // every job's workspace, one after another in m_ws, laid out before any
-  // launch: the groups below run one after another and each job's outputs
-  // (when the caller gave no device pointer) stay in its own region until
-  // they are copied out at the end
+  // every job's workspace, one after another in m_ws, and its outputs in m_out
+  // (the parents of all jobs, then the depths, so that one copy takes them to
+  // the host), laid out before any launch: the groups below run one after
+  // another
   std::vector<JobLayout> L(njobs);
-  std::vector<int64_t> at(njobs + 1, 0);
+  std::vector<int64_t> at(njobs + 1, 0), out_at(njobs + 1, 0);
   for (int j = 0; j < njobs; ++j) {
-    L[j] = job_layout(gs[j]->n, c->tuning.queue_div, true);
+    L[j] = job_layout(gs[j]->n, c->tuning.queue_div, false);
     at[j + 1] = at[j] + L[j].total;
+    out_at[j + 1] = out_at[j] + gs[j]->n;
   }
+  const int64_t total = out_at[njobs];
   if (at[njobs] > c->m_ws_bytes) {
     HIP_TRY(hipStreamSynchronize(c->stream));
     (void)hipFree(c->m_ws);
@@ -2517,52 +2573,94 @@ extern "C" int pbbs_bfs_multi(pbbs_ctx* c, int32_t njobs, pbbs_graph* const* gra
     }
     c->m_ws_bytes = at[njobs];
   }
+  if (2 * total > c->cap_mout) {
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    (void)hipFree(c->m_out);
+    c->m_out = nullptr;
+    c->cap_mout = 0;
+    if (hipMalloc(&c->m_out, 2 * total * sizeof(int32_t)) != hipSuccess) {
+      (void)hipGetLastError();
+      return fail(PBBS_ERR_NOMEM, "multi-graph outputs of %lld entries failed",
+                  (long long)(2 * total));
+    }
+    c->cap_mout = 2 * total;
+  }
   std::vector<int32_t*> dpar(njobs, nullptr), ddep(njobs, nullptr);
   for (int j = 0; j < njobs; ++j) {
-    unsigned char* base = c->m_ws + at[j];
-    dpar[j] = (dev_out && parents && parents[j]) ? parents[j]
-                                                 : reinterpret_cast<int32_t*>(base + L[j].parent);
-    ddep[j] = (dev_out && depths && depths[j]) ? depths[j]
-                                               : reinterpret_cast<int32_t*>(base + L[j].depth);
+    dpar[j] = (dev_out && parents && parents[j]) ? parents[j] : c->m_out + out_at[j];
+    ddep[j] = (dev_out && depths && depths[j]) ? depths[j] : c->m_out + total + out_at[j];
   }
   // A large job runs alone, one launch sequence on the whole device: on its
   // share of a shared grid it takes longer than alone (8 serving graphs of
   // scales 16-22: 2.03 ms in one launch against 1.34 ms one after another),
   // while small graphs gain by sharing (16 graphs of scales 10-17: 4.8x).
-  std::vector<char> alone(njobs, 0);
+  std::vector<char> apart(njobs, 0);
   for (int j = 0; j < njobs; ++j) {
     if (gs[j]->m <= kMultiAloneEdges) continue;
-    alone[j] = 1;
-    int rc = ensure_workspace(c, gs[j]->n);
+    apart[j] = 1;
+    rc = ensure_workspace(c, gs[j]->n);
     if (rc == PBBS_OK)
       rc = gs[j]->off64 ? run_bfs<int64_t>(c, gs[j], sources[j], dpar[j], ddep[j], &stats[j], false)
                         : run_bfs<uint32_t>(c, gs[j], sources[j], dpar[j], ddep[j], &stats[j], false);
     if (rc != PBBS_OK) return rc;
   }
-  // one launch per (offset width, row order) group: jobs of a launch share
-  // the kernel instantiation
+  // one launch per (offset width, row order) group: jobs of a launch share the
+  // kernel instantiation.  Jobs that one workgroup each can run take a launch
+  // of those where every job is such (one per offset width); beside larger
+  // jobs they take their share of the persistent grid, where they are done
+  // before the others (16 graphs of scales 10-17: 480 us a call, 570 with the
+  // smaller ones in a launch ahead).
+  bool all_small = true;
+  for (int j = 0; j < njobs; ++j) all_small = all_small && want_small(c, gs[j], false);
   for (int off64 = 0; off64 < 2; ++off64) {
+    if (all_small) {
+      std::vector<int> ids;
+      for (int j = 0; j < njobs; ++j)
+        if ((int)gs[j]->off64 == off64) ids.push_back(j);
+      if (!ids.empty())
+        rc = run_multi_small(c, c->m_host_params + off64, c->m_params + off64, ids, gs, sources,
+                             dpar, ddep, stats, off64);
+      if (rc != PBBS_OK) return rc;
+      continue;
+    }
     for (int sorted = 0; sorted < 2; ++sorted) {
       std::vector<int> ids;
       for (int j = 0; j < njobs; ++j)
-        if (!alone[j] && (int)gs[j]->off64 == off64 && (int)gs[j]->sorted == sorted)
+        if (!apart[j] && (int)gs[j]->off64 == off64 && (int)gs[j]->sorted == sorted)
           ids.push_back(j);
       if (ids.empty()) continue;
-      const int rc =
-          off64 ? run_multi_group<int64_t>(c, ids, gs, sources, L, at, dpar, ddep, stats, sorted)
-                : run_multi_group<uint32_t>(c, ids, gs, sources, L, at, dpar, ddep, stats, sorted);
+      const int slot = 2 + 2 * off64 + sorted;
+      rc = off64 ? run_multi_group<int64_t>(c, c->m_host_params + slot, c->m_params + slot, ids,
+                                            gs, sources, L, at, dpar, ddep, stats, sorted)
+                 : run_multi_group<uint32_t>(c, c->m_host_params + slot, c->m_params + slot, ids,
+                                             gs, sources, L, at, dpar, ddep, stats, sorted);
       if (rc != PBBS_OK) return rc;
     }
   }
-  if (!dev_out) {
+  if (!dev_out && (parents || depths)) {
+    // one copy to pinned memory, then to the caller's arrays (a copy to
+    // pageable memory for each took 17 us a job and array)
+    const int64_t lo = parents ? 0 : total, hi = depths ? 2 * total : total;
+    int32_t* p = ensure_pinned(c, hi - lo);
+    if (p) {
+      HIP_TRY(hipMemcpyAsync(p, c->m_out + lo, (hi - lo) * sizeof(int32_t), hipMemcpyDeviceToHost,
+                             c->stream));
+      HIP_TRY(hipStreamSynchronize(c->stream));
+    }
     for (int j = 0; j < njobs; ++j) {
       const size_t bytes = (size_t)gs[j]->n * sizeof(int32_t);
-      if (parents && parents[j])
-        HIP_TRY(hipMemcpyAsync(parents[j], dpar[j], bytes, hipMemcpyDeviceToHost, c->stream));
-      if (depths && depths[j])
-        HIP_TRY(hipMemcpyAsync(depths[j], ddep[j], bytes, hipMemcpyDeviceToHost, c->stream));
+      int32_t* const out[2] = {parents ? parents[j] : nullptr, depths ? depths[j] : nullptr};
+      for (int k = 0; k < 2; ++k) {
+        if (!out[k]) continue;
+        const int64_t from = k * total + out_at[j];
+        if (p)
+          std::memcpy(out[k], p + (from - lo), bytes);
+        else
+          HIP_TRY(hipMemcpyAsync(out[k], c->m_out + from, bytes, hipMemcpyDeviceToHost,
+                                 c->stream));
+      }
     }
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    if (!p) HIP_TRY(hipStreamSynchronize(c->stream));
   }
   return PBBS_OK;
 }
