@@ -70,7 +70,27 @@ struct BfsState {
 // scans), sorted rows read from the CSR, sorted rows with row-top records;
 // and any-parent levels (bottom-up rows probed from their smallest entry up,
 // the first frontier neighbour found taken as the parent, sorted or not).
-enum LevelVariant { kLevelUnsorted = 0, kLevelSorted = 1, kLevelSortedTops = 2, kLevelAnyParent = 3 };
+// kLevelStream: sorted rows with records, on graphs where a small frontier of
+// hubs may meet most of the edges (levels that stream the adjacency; kept out of
+// the other variants, whose levels they slow by 1 to 2%).
+enum LevelVariant {
+  kLevelUnsorted = 0,
+  kLevelSorted = 1,
+  kLevelSortedTops = 2,
+  kLevelAnyParent = 3,
+  kLevelStream = 4
+};
+
+// A streaming level's limits (bfs_kernels.hip: bu_stream).
+// Vertices of F_k that leave its hashed bit set sparse: 13722 take 813 us
+// against the general level's 747.
+constexpr unsigned kStreamMax = 8192;
+// Below these entries a level takes some tens of microseconds either way.
+constexpr long long kStreamMinM = 1ll << 26;
+// Streaming costs 1.2 ps an entry of the graph, top-down 57 ps an edge of F_k
+// (rMat 2^24, 15M edges: 884 us; 2^22, 4.5M: 257), so they meet at a 48th of m;
+// the line is at m / (kStreamTd * td_to_bu_div), a 40th by default.
+constexpr unsigned kStreamTd = 2;
 
 // Everything a level kernel needs.  The init kernel copies it into device
 // memory so one captured HIP graph of level launches serves every run that

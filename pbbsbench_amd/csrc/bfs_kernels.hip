@@ -869,6 +869,211 @@ __device__ void bottom_up(const LevelView<OffT>& a, StageBuf& sb, Stage& stg, Bu
     bu_finish_parked<OffT, kAsc>(a, sb, stg, L, npark, kTops && !kAsc ? kTopEntries : 4);
 }
 
+// A bottom-up level with a small frontier of large degree sum (the hubs of a
+// skewed graph): nearly every row is read to its end, and a bitmap lookup for
+// each entry occupies a CU's address unit for a cycle.  Here the adjacency is
+// streamed in order, 16 bytes a lane, and every entry first meets a hashed bit
+// set of F_k in LDS; the few that pass (members, and |F_k| in kStreamBits of
+// the others) are listed, looked up in the bitmap 128 at a time and claim their
+// row by an LDS max.  The work axis is the entries plus kStreamCost for each
+// group of rows, cut evenly; what a cut divides is combined in memory.
+// Bound by the loads in flight (3.4 TB/s): rMat 2^24, 520M entries, |F_2| 4538:
+// 1122 -> 642 us; 2275 (top-down before): 884 -> 610; 2^22, 128M, 988: 257 ->
+// 160.  Groups of 64 rows 735, four loads ahead (3 wavefronts a SIMD) 735; a
+// cost of 512, 2048 or 4096 for a group 846, 683 or 761 us.
+constexpr int kStreamBits = 1 << 17;
+constexpr int kStreamRows = 4;                // rows of a group per lane
+constexpr int kStreamGroup = kStreamRows * kWave;
+constexpr int kStreamCost = 1024;             // of a group on the work axis
+constexpr int kStreamList = 2 * kWave;        // entries checked together
+constexpr int kStreamUnroll = 2;              // 16-byte loads in flight per lane
+
+__device__ __forceinline__ unsigned stream_hash(int u) {
+  return (unsigned)__mul24(u, 0x9E3779) >> 15;   // 17 bits, of the low 24
+}
+
+template <typename OffT>
+__device__ void bu_stream(const LevelView<OffT>& a, StageBuf& sb, Stage& stg, BuLds<OffT>& L,
+                          const unsigned long long (&qc)[kSubQueues]) {
+  constexpr int kListCap = kStreamList + kWave;
+  static_assert(sizeof(L) >= kStreamBits / 8 && kWaveBuf > kListCap + kStreamGroup,
+                "LDS of the other levels");
+  static_assert(kStreamList == 2 * kWave, "two groups a check");
+  typedef int i32x4 __attribute__((ext_vector_type(4)));
+  unsigned* filter = reinterpret_cast<unsigned*>(&L);
+  const int w = threadIdx.x / kWave;
+  const unsigned lane = lane_id();
+  for (int i = threadIdx.x; i < kStreamBits / 32; i += kBlock) filter[i] = 0;
+  int32_t* list_u = sb.v[w];                // entries that passed: neighbour, position
+  uint32_t* list_e = sb.eo[w];
+  int32_t* best = sb.v[w] + kListCap;       // the group's parents; INT_MAX: reached before
+  uint32_t* rows = sb.eo[w] + kListCap;     // its row starts, and the end of the last
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < kSubQueues; ++s) {
+    const gptr<const int32_t> q = a.q_cur + s * a.qcap;
+    for (unsigned i = threadIdx.x; i < (unsigned)qc[s]; i += kBlock) {
+      const unsigned h = stream_hash(q[i]);
+      atomicOr(&filter[h >> 5], 1u << (h & 31));
+    }
+  }
+  __syncthreads();
+  const gptr<const unsigned long long> fbc64 = (gptr<const unsigned long long>)a.fb_cur;
+  const long long groups = (a.n + kStreamGroup - 1) / kStreamGroup;
+  const long long X = a.m + (long long)kStreamCost * groups;
+  const long long x0 = (long long)((unsigned long long)X * a.gw / a.W);
+  const long long x1 = (long long)((unsigned long long)X * (a.gw + 1) / a.W);
+  // the last group that starts at or before x0, 64 tries a step
+  long long lo = 0, hi = groups;
+  while (hi - lo > 1) {
+    const long long step = (hi - lo + kWave - 1) / kWave;
+    const long long i = lo + lane * step;
+    const bool le = i < hi && (long long)a.off[i * kStreamGroup] + kStreamCost * i <= x0;
+    const unsigned c = (unsigned)__popcll(__ballot(le));   // >= 1: group lo is
+    lo += (c - 1) * step;
+    hi = min(hi, lo + step);
+  }
+  // a group's rows and masks, loaded one group ahead
+  uint32_t ns[kStreamRows], nend = 0;
+  unsigned long long nold = 0, nfk = 0;
+  auto load_group = [&](long long g) {
+    const long long v = g * kStreamGroup + lane;
+#pragma unroll
+    for (int q = 0; q < kStreamRows; ++q) ns[q] = (uint32_t)a.off[min(v + q * kWave, a.n)];
+    nend = (uint32_t)a.off[min((g + 1) * kStreamGroup, a.n)];
+    const long long word = min(g * kStreamRows + (long long)min(lane, (unsigned)kStreamRows - 1),
+                               a.nwords - 1);
+    nold = a.visited[word];
+    nfk = fbc64[word];
+  };
+  load_group(lo);
+  for (long long g = lo; g < groups; ++g) {
+    uint32_t s[kStreamRows];
+#pragma unroll
+    for (int q = 0; q < kStreamRows; ++q) s[q] = ns[q];
+    const unsigned long long old = nold, vis = nold | nfk;
+    const uint32_t o0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)s[0]);
+    const uint32_t o1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)nend);
+    const long long cost = (long long)kStreamCost * g;
+    if ((long long)o0 + cost >= x1) break;
+    load_group(g + 1);
+    const bool mine = lane < (unsigned)kStreamRows && g * kStreamRows + lane < a.nwords;
+    if (mine && vis != old) a.visited[g * kStreamRows + lane] = vis;   // F_k folded in
+    const long long c0 = max((long long)o0, x0 - cost), c1 = min((long long)o1, x1 - cost);
+    if (c0 >= c1 || !__ballot(mine && ~vis != 0ull)) continue;
+    const uint32_t e0 = (uint32_t)c0, e1 = (uint32_t)c1, b0 = e0 & ~3u;
+    const bool cut = e0 > o0 || e1 < o1;
+#pragma unroll
+    for (int q = 0; q < kStreamRows; ++q) {
+      const unsigned long long word = g * kStreamRows + q < a.nwords ? __shfl(vis, q) : ~0ull;
+      best[q * kWave + lane] = word >> lane & 1ull ? INT_MAX : -1;
+      rows[q * kWave + lane] = s[q];
+    }
+    if (lane == 0) rows[kStreamGroup] = o1;
+    unsigned n = 0;   // entries listed
+    auto check = [&]() {   // the first kStreamList of them
+      wave_lds_sync();
+      int u[2];
+      uint32_t e[2];
+      bool hit[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        u[t] = t * kWave + lane < n ? list_u[t * kWave + lane] : -1;
+        e[t] = list_e[t * kWave + lane];
+        hit[t] = in_set_or_none(a.fb_cur, u[t]);
+      }
+      int row[2] = {0, 0};   // the last row that starts at or before e
+#pragma unroll
+      for (int st = kStreamGroup / 2; st >= 1; st >>= 1)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          if (rows[row[t] + st] <= e[t]) row[t] += st;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        if (hit[t]) atomicMax(&best[row[t]], u[t]);
+      const unsigned rest = n > (unsigned)kStreamList ? n - kStreamList : 0u;   // < 64
+      const int tu = list_u[kStreamList + lane];
+      const uint32_t te = list_e[kStreamList + lane];
+      wave_lds_sync();
+      if (lane < rest) {
+        list_u[lane] = tu;
+        list_e[lane] = te;
+      }
+      n = rest;
+    };
+    // entries are loaded a step ahead
+    constexpr uint32_t kStep = 4 * kWave * kStreamUnroll;
+    i32x4 c[kStreamUnroll], d[kStreamUnroll];
+    auto load_step = [&](uint32_t b, i32x4 (&r)[kStreamUnroll]) {
+#pragma unroll
+      for (int t = 0; t < kStreamUnroll; ++t) {
+        // the last entries' load may reach kAdjPad past the graph's end
+        const uint32_t i = b + (uint32_t)(4 * kWave * t) + 4 * lane;
+        r[t] = *(gptr<const i32x4>)(a.adj + (i < e1 ? i : b0));
+      }
+    };
+    load_step(b0, c);
+    for (uint32_t at = 0; at < e1 - b0; at += kStep) {
+      const uint32_t b = b0 + at;
+      if (e1 - b > kStep) load_step(b + kStep, d);
+      if (b < e0 || e1 - b < kStep) {   // entries outside the share: no vertex
+#pragma unroll
+        for (int j = 0; j < 4 * kStreamUnroll; ++j) {
+          const uint32_t e = b + (uint32_t)(4 * kWave * (j / 4) + j % 4) + 4 * lane;
+          if (e - e0 >= e1 - e0) c[j / 4][j % 4] = -1;
+        }
+      }
+      unsigned f[4 * kStreamUnroll];
+#pragma unroll
+      for (int j = 0; j < 4 * kStreamUnroll; ++j) {
+        const unsigned h = stream_hash(c[j / 4][j % 4]);
+        f[j] = filter[h >> 5] >> (h & 31);
+      }
+#pragma unroll
+      for (int j = 0; j < 4 * kStreamUnroll; ++j) {
+        const bool pass = f[j] & 1u;
+        const unsigned long long pm = __ballot(pass);
+        if (!pm) continue;
+        if (pass) {
+          const unsigned slot = n + lanes_below(pm);   // n < kStreamList
+          list_u[slot] = c[j / 4][j % 4];
+          list_e[slot] = b + (uint32_t)(4 * kWave * (j / 4) + j % 4) + 4 * lane;
+        }
+        n += (unsigned)__popcll(pm);
+        if (n >= (unsigned)kStreamList) check();
+      }
+#pragma unroll
+      for (int t = 0; t < kStreamUnroll; ++t) c[t] = d[t];
+    }
+    if (n) check();
+    wave_lds_sync();
+#pragma unroll
+    for (int q = 0; q < kStreamRows; ++q) {
+      const int found = best[q * kWave + lane];
+      const bool hit = found >= 0 && found != INT_MAX;
+      unsigned long long fresh = __ballot(hit);
+      if (!fresh) continue;
+      const long long word = g * kStreamRows + q;
+      const int v = (int)(word * kWave + lane);
+      if (hit) {
+        if (cut) atomicMax(gen(&a.parent[v]), found);
+        else a.parent[v] = found;
+        a.depth[v] = a.k + 1;
+      }
+      if (cut) {
+        unsigned long long was = 0;
+        if (lane == 0) was = atomicOr(gen(&a.fb_next[word]), fresh);
+        fresh &= ~__shfl(was, 0);
+      } else if (lane == 0) {
+        a.fb_next[word] = fresh;
+      }
+      stage_count(stg, fresh >> lane & 1ull,
+                  rows[q * kWave + lane + 1] - rows[q * kWave + lane]);
+    }
+    wave_lds_sync();   // before the next group's rows
+  }
+}
+
 // A top-down level after a bottom-up one: F_k exists only as its bitmap.
 // Each wavefront takes an equal share of the bitmap words, gathers its
 // frontier vertices 64 at a time (one per lane, with row start and degree)
@@ -938,6 +1143,16 @@ __device__ __forceinline__ int level_mode(const BfsArgs<OffT>& A, int prev, unsi
   return ((long long)cnt > A.n / A.bu_to_td_div) ? kBottomUp : kTopDown;
 }
 
+// Whether bu_stream takes the level: F_k is small and known by its queue (the
+// level before was top-down), and top-down would take longer.
+template <typename OffT>
+__device__ __forceinline__ bool stream_level(const BfsArgs<OffT>& A, int prev,
+                                             unsigned long long cnt, unsigned long long E) {
+  return prev == kTopDown && A.symmetric && A.td_to_bu_div > 0 && cnt <= kStreamMax &&
+         A.m >= kStreamMinM &&
+         E * (unsigned)A.td_to_bu_div * kStreamTd > (unsigned long long)A.m;
+}
+
 // Level k of the BFS, as workgroup vb of a grid of vg workgroups (the
 // launch's own grid, or this BFS's part of a launch shared with others).
 // Returns false if F_k is empty (the BFS is over), true once this
@@ -996,7 +1211,8 @@ __device__ void rebuild_bitmaps(const BfsArgs<OffT>* __restrict__ A, const int k
   }
 }
 
-template <typename OffT, bool kSorted, bool kTops, bool kLazy = false, bool kAsc = false>
+template <typename OffT, bool kSorted, bool kTops, bool kLazy = false, bool kAsc = false,
+          bool kStream = false>
 __device__ __forceinline__ bool level_step(const BfsArgs<OffT>* __restrict__ A, const int k,
                                            StageBuf& sb, BuLds<OffT>& bl, const unsigned vb,
                                            const unsigned vg, LazyBitmaps* lz = nullptr) {
@@ -1031,8 +1247,13 @@ __device__ __forceinline__ bool level_step(const BfsArgs<OffT>* __restrict__ A, 
     return false;
   }
   const int prev = k == 0 ? kTopDown : st->modes[(k - 1) & 3];
-  const int mode = level_mode(*A, prev, cnt, E);
+  int mode = level_mode(*A, prev, cnt, E);
   const bool qover = st->qover[c0] != 0;
+  bool stream = false;
+  if constexpr (kStream) {
+    stream = stream_level(*A, prev, cnt, E) && !qover;
+    if (stream) mode = kBottomUp;
+  }
   bool keep = true;   // this level keeps the bitmaps
   if constexpr (kLazy) {
     if (lz->on) {
@@ -1121,7 +1342,10 @@ __device__ __forceinline__ bool level_step(const BfsArgs<OffT>* __restrict__ A, 
   } else
   {
     slot_priority(A->num_cus);   // bottom-up only: top-down levels measured the same with it
-    bottom_up<OffT, kSorted, kTops, kAsc>(a, sb, stg, bl);
+    if (kStream && stream)
+      bu_stream(a, sb, stg, bl, qc);
+    else
+      bottom_up<OffT, kSorted, kTops, kAsc>(a, sb, stg, bl);
     __builtin_amdgcn_s_setprio(0);
   }
   stage_flush_block(a, sb, stg, mode == kTopDown);
@@ -1130,12 +1354,13 @@ __device__ __forceinline__ bool level_step(const BfsArgs<OffT>* __restrict__ A, 
 
 // One level per launch: the level number comes from the workgroup's own
 // counter, so a captured sequence of launches needs no host input.
-template <typename OffT, bool kSorted, bool kTops, bool kAsc = false>
+template <typename OffT, bool kSorted, bool kTops, bool kAsc = false, bool kStream = false>
 __global__ __launch_bounds__(kBlock) void bfs_level_kernel(const BfsArgs<OffT>* __restrict__ A) {
   __shared__ StageBuf sb;
   __shared__ BuLds<OffT> bl;
   const int k = (int)A->wg_level[blockIdx.x];
-  if (level_step<OffT, kSorted, kTops, false, kAsc>(A, k, sb, bl, blockIdx.x, gridDim.x) &&
+  if (level_step<OffT, kSorted, kTops, false, kAsc, kStream>(A, k, sb, bl, blockIdx.x,
+                                                             gridDim.x) &&
       threadIdx.x == 0)
     A->wg_level[blockIdx.x] = (uint32_t)(k + 1);
 }
@@ -2526,6 +2751,8 @@ const void* level_kernel_symbol(int variant) {
   switch (variant) {
     case kLevelAnyParent:
       return reinterpret_cast<const void*>(&bfs_level_kernel<OffT, true, false, true>);
+    case kLevelStream:
+      return reinterpret_cast<const void*>(&bfs_level_kernel<OffT, true, true, false, true>);
     case kLevelSortedTops: return reinterpret_cast<const void*>(&bfs_level_kernel<OffT, true, true>);
     case kLevelSorted: return reinterpret_cast<const void*>(&bfs_level_kernel<OffT, true, false>);
     default: return reinterpret_cast<const void*>(&bfs_level_kernel<OffT, false, false>);
@@ -2589,6 +2816,9 @@ hipError_t launch_bfs_level(const BfsArgs<OffT>* dargs, int variant, int grid, h
   if (variant == kLevelAnyParent)
     hipLaunchKernelGGL((bfs_level_kernel<OffT, true, false, true>), dim3(grid), dim3(kBlock), 0,
                        stream, dargs);
+  else if (variant == kLevelStream)
+    hipLaunchKernelGGL((bfs_level_kernel<OffT, true, true, false, true>), dim3(grid), dim3(kBlock),
+                       0, stream, dargs);
   else if (variant == kLevelSortedTops)
     hipLaunchKernelGGL((bfs_level_kernel<OffT, true, true>), dim3(grid), dim3(kBlock), 0, stream, dargs);
   else if (variant == kLevelSorted)

@@ -1113,6 +1113,16 @@ static int level_variant(const pbbs_graph* g, const uint32_t* tops) {
   return !g->sorted ? kLevelUnsorted : tops ? kLevelSortedTops : kLevelSorted;
 }
 
+// The variant of a run with a launch per level: streaming levels where
+// kStreamMax vertices can have the edges that start one.
+static int launch_variant(const pbbs_ctx* c, const pbbs_graph* g, int variant) {
+  const bool stream = variant == kLevelSortedTops && g->symmetric && g->m >= kStreamMinM &&
+                      c->tuning.td_to_bu_div > 0 &&
+                      (double)kStreamMax * g->max_degree * kStreamTd * c->tuning.td_to_bu_div >
+                          (double)g->m;
+  return stream ? (int)kLevelStream : variant;
+}
+
 // Workgroups of the persistent kernel that fit on the device at once.
 static int persist_capacity(pbbs_ctx* c, bool off64, int variant) {
   int per_cu = 0;
@@ -1211,8 +1221,8 @@ static int begin_bfs(pbbs_ctx* c, pbbs_graph* g, int32_t s, int32_t* d_parent, i
   const uint32_t* tops = nullptr;
   int rc = any_parent ? PBBS_OK : ensure_tops<OffT>(c, g, &tops, own);
   if (rc != PBBS_OK) return rc;
-  const int variant = any_parent ? kLevelAnyParent : level_variant(g, tops);
-  int grid = level_grid(c, g->off64, variant);
+  int variant = any_parent ? kLevelAnyParent : level_variant(g, tops);
+  int grid = 0;
   bool persist = false, deep = false;
   DeepWs dws{};
   if (allow_persist && want_deep(c, g, own, any_parent)) {
@@ -1228,6 +1238,10 @@ static int begin_bfs(pbbs_ctx* c, pbbs_graph* g, int32_t s, int32_t* d_parent, i
       persist = true;
       grid = persist_grid(c, cap);
     }
+  }
+  if (!persist) {
+    variant = launch_variant(c, g, variant);
+    grid = level_grid(c, g->off64, variant);
   }
   const uint32_t* bounds = nullptr;
   if (!deep) {   // the deep path has no bottom-up levels
@@ -1709,7 +1723,7 @@ static int run_profile(pbbs_ctx* c, pbbs_graph* g, int32_t s, pbbs_level_profile
   const uint32_t* tops = nullptr;
   int brc = ensure_tops<OffT>(c, g, &tops);
   if (brc != PBBS_OK) return brc;
-  const int variant = level_variant(g, tops);
+  const int variant = launch_variant(c, g, level_variant(g, tops));
   const int grid = level_grid(c, g->off64, variant);
   const uint32_t* bounds = nullptr;
   brc = ensure_bounds(c, g, (int64_t)grid * kWavesPerBlock, &bounds);
@@ -1810,7 +1824,7 @@ static int prepare_graph(pbbs_ctx* c, pbbs_graph* g, uint32_t what) {
     int rc = ensure_tops<OffT>(c, g, &tops);
     if (rc != PBBS_OK) return rc;
     const int variant = level_variant(g, tops);
-    const int grid = level_grid(c, g->off64, variant);
+    const int grid = level_grid(c, g->off64, launch_variant(c, g, variant));
     const uint32_t* bounds = nullptr;
     rc = ensure_bounds(c, g, (int64_t)grid * kWavesPerBlock, &bounds);
     if (rc != PBBS_OK) return rc;
