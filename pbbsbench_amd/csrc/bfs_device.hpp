@@ -215,7 +215,6 @@ struct MbfsArgs {
   MbfsState* st;
   uint32_t* wg_level;
   int32_t* host_status;
-  const int32_t* sources;      // [nsrc]
   const int32_t* pull_rows;    // first list entry of each wavefront's pull slice (waves + 1)
   const int32_t* rows;         // vertices of degree > 0, ascending
   int64_t nrows;
@@ -231,6 +230,11 @@ struct MbfsArgs {
   int32_t preset_parents;      // 1: parent already holds -1 everywhere (filled ahead of
                                // the batch), so the clear kernel leaves it alone
   int32_t pad;
+};
+
+// A batch's sources, as its seed launch takes them.
+struct BatchSources {
+  int32_t v[kMaxSources];
 };
 
 // ------------------------------------------------- maximal independent set

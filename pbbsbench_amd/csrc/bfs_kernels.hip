@@ -2404,13 +2404,14 @@ hipError_t launch_fill_minus1(int32_t* p, long long count, int grid, hipStream_t
 // One workgroup: marks the sources, queues the distinct ones as F_0 and
 // resets the control block.
 template <typename OffT>
-__global__ __launch_bounds__(kBlock) void mbfs_seed_kernel(MbfsArgs<OffT> a, MbfsArgs<OffT>* dst) {
+__global__ __launch_bounds__(kBlock) void mbfs_seed_kernel(MbfsArgs<OffT> a, MbfsArgs<OffT>* dst,
+                                                           BatchSources sources) {
   __shared__ int first[kMaxSources];
   __shared__ int src[kMaxSources];
   __shared__ unsigned long long deg[kMaxSources];
   const int t = threadIdx.x;
   if (t < a.nsrc) {
-    const int s = a.sources[t];
+    const int s = sources.v[t];
     src[t] = s;
     deg[t] = (unsigned long long)(a.off[s + 1] - a.off[s]);
     const unsigned long long bit = 1ull << t;
@@ -2459,7 +2460,9 @@ __global__ __launch_bounds__(kBlock) void mbfs_seed_kernel(MbfsArgs<OffT> a, Mbf
 // the level table (n where source i never reached v; entries from
 // kDepthEscape on were written during the levels).  A lane takes 4
 // consecutive vertices, so each source's store is 16 bytes per lane and 1 KB
-// per wavefront.
+// per wavefront.  Launched behind every chunk of levels, and done at once
+// unless they ended the BFS: the host need not see the end first (30 to 40 us
+// of an idle device; 12 sources on rMat 2^18: 312 -> 292 us a batch).
 template <typename OffT>
 __global__ __launch_bounds__(kBlock) void mbfs_depth_kernel(MbfsArgs<OffT> a) {
   // A workgroup takes tiles of 256 vertices: their 64-byte depth rows are
@@ -2470,6 +2473,7 @@ __global__ __launch_bounds__(kBlock) void mbfs_depth_kernel(MbfsArgs<OffT> a) {
   static_assert(kWavesPerBlock * 16 == kMaxSources, "four wavefronts of 16 sources each");
   __shared__ uint32_t rows[kBlock * kRowDw];
   __shared__ unsigned long long rvm_lds[kBlock];
+  if (!a.st->finished) return;
   const gptr<const unsigned long long> vis = glob((const unsigned long long*)a.vis);
   const gptr<const u32x4> dl = glob((const u32x4*)a.dlev);
   const gptr<int32_t> depth = glob(a.depth);
@@ -2903,12 +2907,13 @@ hipError_t launch_row_tops(const OffT* off, const int32_t* adj, long long n, uin
 }
 
 template <typename OffT>
-hipError_t launch_mbfs_setup(const MbfsArgs<OffT>& a, MbfsArgs<OffT>* dst, int grid,
-                             hipStream_t stream) {
+hipError_t launch_mbfs_setup(const MbfsArgs<OffT>& a, MbfsArgs<OffT>* dst,
+                             const BatchSources& sources, int grid, hipStream_t stream) {
   hipLaunchKernelGGL(mbfs_clear_kernel<OffT>, dim3(grid), dim3(kBlock), 0, stream, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(mbfs_seed_kernel<OffT>, dim3(1), dim3(kBlock), 0, stream, a, dst);
+  hipLaunchKernelGGL(mbfs_seed_kernel<OffT>, dim3(1), dim3(kBlock), 0, stream, a, dst,
+                     sources);
   return hipGetLastError();
 }
 
@@ -3027,8 +3032,8 @@ hipError_t launch_mbfs_depth(const MbfsArgs<OffT>& a, int grid, hipStream_t stre
                                                  hipStream_t);                                   \
   template hipError_t launch_graph_rows<OffT>(const OffT*, const int32_t*, long long, long long, \
                                               unsigned long long*, int, hipStream_t);            \
-  template hipError_t launch_mbfs_setup<OffT>(const MbfsArgs<OffT>&, MbfsArgs<OffT>*, int,      \
-                                             hipStream_t);                                      \
+  template hipError_t launch_mbfs_setup<OffT>(const MbfsArgs<OffT>&, MbfsArgs<OffT>*,           \
+                                             const BatchSources&, int, hipStream_t);            \
   template const void* mbfs_level_symbol<OffT>(bool);                                           \
   template hipError_t launch_mbfs_level<OffT>(const MbfsArgs<OffT>*, bool, int, hipStream_t);    \
   template hipError_t launch_pull_rows<OffT>(const OffT*, const int32_t*, long long, long long,  \

@@ -58,8 +58,8 @@ template <typename OffT>
 hipError_t launch_graph_rows(const OffT* off, const int32_t* adj, long long n, long long m,
                              unsigned long long* counters, int grid, hipStream_t stream);
 template <typename OffT>
-hipError_t launch_mbfs_setup(const MbfsArgs<OffT>& a, MbfsArgs<OffT>* dst, int grid,
-                             hipStream_t stream);
+hipError_t launch_mbfs_setup(const MbfsArgs<OffT>& a, MbfsArgs<OffT>* dst,
+                             const BatchSources& sources, int grid, hipStream_t stream);
 template <typename OffT>
 const void* mbfs_level_symbol(bool sorted);
 template <typename OffT>
@@ -193,7 +193,6 @@ struct pbbs_ctx {
     int K = 0;
     int64_t launched = 0;
     int64_t limit = 0;
-    bool finalized = false;  // batched: the depth pass after the last level is queued
     bool persist = false;    // single source: every level in one persistent launch
     bool token = false;      // holds the device's persistent-launch token
     bool any_parent = false; // single source: PBBS_BFS_ANY_PARENT levels
@@ -215,7 +214,6 @@ struct pbbs_ctx {
   MbfsState* b_state = nullptr;
   MbfsState* b_host_state = nullptr;     // pinned: the control block after the depth pass
   void* b_args = nullptr;                // device copy of MbfsArgs<OffT>
-  int32_t* b_sources = nullptr;          // kMaxSources
   int64_t cap_bout = 0;                  // int32 entries of each output buffer
   int32_t* b_parent = nullptr;          // parents of the last batched run
   int32_t* b_depth = nullptr;
@@ -550,7 +548,6 @@ int pbbs_ctx_destroy(pbbs_ctx* c) {
   (void)hipFree(c->b_state);
   if (c->b_host_state) (void)hipHostFree(c->b_host_state);
   (void)hipFree(c->b_args);
-  (void)hipFree(c->b_sources);
   (void)hipFree(c->b_parent);
   (void)hipFree(c->b_parent_alt);
   (void)hipFree(c->b_depth);
@@ -1033,6 +1030,17 @@ static int launch_chunk(pbbs_ctx* c) {
     }
   }
   r.launched += r.K;
+  if (r.kind == 1) {   // the depth outputs and totals, if these levels ended the BFS
+    const int grid = std::max(1, c->num_cus * 8);
+    if (r.off64)
+      HIP_TRY(launch_mbfs_depth<int64_t>(*reinterpret_cast<MbfsArgs<int64_t>*>(c->b_last_args),
+                                         grid, c->stream));
+    else
+      HIP_TRY(launch_mbfs_depth<uint32_t>(*reinterpret_cast<MbfsArgs<uint32_t>*>(c->b_last_args),
+                                          grid, c->stream));
+    HIP_TRY(hipMemcpyAsync(c->b_host_state, c->b_state, sizeof(MbfsState), hipMemcpyDeviceToHost,
+                           c->stream));
+  }
   HIP_TRY(hipEventRecord(c->ev_end, c->stream));
   return PBBS_OK;
 }
@@ -1051,22 +1059,6 @@ static int poll_run_impl(pbbs_ctx* c, bool wait, bool* done) {
   }
   if (c->host_status[0]) {
     pbbs_ctx::Run& r = c->run;
-    if (r.kind == 1 && !r.finalized) {
-      // batched: write the depth outputs, then report done once that is through
-      const int grid = std::max(1, c->num_cus * 8);
-      if (r.off64)
-        HIP_TRY(launch_mbfs_depth<int64_t>(
-            *reinterpret_cast<MbfsArgs<int64_t>*>(c->b_last_args), grid, c->stream));
-      else
-        HIP_TRY(launch_mbfs_depth<uint32_t>(
-            *reinterpret_cast<MbfsArgs<uint32_t>*>(c->b_last_args), grid, c->stream));
-      HIP_TRY(hipMemcpyAsync(c->b_host_state, c->b_state, sizeof(MbfsState),
-                             hipMemcpyDeviceToHost, c->stream));
-      HIP_TRY(hipEventRecord(c->ev_end, c->stream));
-      r.finalized = true;
-      if (!wait) return PBBS_OK;
-      HIP_TRY(hipEventSynchronize(c->ev_end));
-    }
     if (r.graph) r.graph->last_launches[r.kind] = c->host_status[1] + 1;
     release_persist(c);
     r.persist = false;
@@ -1263,7 +1255,6 @@ static int begin_bfs(pbbs_ctx* c, pbbs_graph* g, int32_t s, int32_t* d_parent, i
   r.K = first_chunk(c, g, r.kind);
   r.graph = g;
   r.launched = 0;
-  r.finalized = false;
   r.limit = g->n + 2;
   r.persist = persist;
   r.any_parent = any_parent;
@@ -1865,25 +1856,21 @@ extern "C" int pbbs_graph_prepare(pbbs_ctx* c, pbbs_graph* g, uint32_t what, dou
 // --------------------------------------------------------------- batched BFS
 static int ensure_batch_workspace(pbbs_ctx* c, int64_t n, int64_t out_entries, bool need_out) {
   if (!c->b_state) {
-    // all four control buffers or none: b_state marks the set as present
+    // all three control buffers or none: b_state marks the set as present
     MbfsState* st = nullptr;
     MbfsState* hst = nullptr;
     void* args = nullptr;
-    int32_t* src = nullptr;
     if (hipMalloc(&st, sizeof(MbfsState)) != hipSuccess ||
         hipHostMalloc((void**)&hst, sizeof(MbfsState), hipHostMallocDefault) != hipSuccess ||
-        hipMalloc(&args, sizeof(MbfsArgs<int64_t>)) != hipSuccess ||
-        hipMalloc(&src, kMaxSources * sizeof(int32_t)) != hipSuccess) {
+        hipMalloc(&args, sizeof(MbfsArgs<int64_t>)) != hipSuccess) {
       (void)hipGetLastError();
       (void)hipFree(st);
       if (hst) (void)hipHostFree(hst);
       (void)hipFree(args);
-      (void)hipFree(src);
       return fail(PBBS_ERR_NOMEM, "batched control buffers failed");
     }
     c->b_host_state = hst;
     c->b_args = args;
-    c->b_sources = src;
     c->b_state = st;
   }
   if (n > c->cap_bn) {
@@ -1983,8 +1970,8 @@ static int get_batch_graph(pbbs_ctx* c, bool sorted, int grid, int K, hipGraphEx
 // are ignored), which lets the parents come pre-filled with -1 (see
 // b_parent_alt); otherwise the clear kernel fills the caller's parents.
 template <typename OffT>
-static int begin_batch(pbbs_ctx* c, pbbs_graph* g, int32_t nsrc, int32_t* d_parent,
-                       int32_t* d_depth, bool own_out) {
+static int begin_batch(pbbs_ctx* c, pbbs_graph* g, const int32_t* sources, int32_t nsrc,
+                       int32_t* d_parent, int32_t* d_depth, bool own_out) {
   const int64_t n = g->n;
   const int64_t entries = (int64_t)nsrc * n;
   bool preset = false;
@@ -2015,7 +2002,6 @@ static int begin_batch(pbbs_ctx* c, pbbs_graph* g, int32_t nsrc, int32_t* d_pare
   a.st = c->b_state;
   a.wg_level = c->w_wg_level;
   a.host_status = c->host_status;
-  a.sources = c->b_sources;
   a.n = n;
   a.m = g->m;
   a.nwords = (n + kWave - 1) / kWave;
@@ -2045,7 +2031,6 @@ static int begin_batch(pbbs_ctx* c, pbbs_graph* g, int32_t nsrc, int32_t* d_pare
   r.K = first_chunk(c, g, r.kind);
   r.graph = g;
   r.launched = 0;
-  r.finalized = false;
   r.limit = n + 2;
   const int setup_grid =
       (int)std::max<int64_t>(1, std::min<int64_t>((n + kBlock - 1) / kBlock, c->num_cus * 16));
@@ -2059,7 +2044,9 @@ static int begin_batch(pbbs_ctx* c, pbbs_graph* g, int32_t nsrc, int32_t* d_pare
   hs[1] = 0;
   HIP_TRY(hipEventRecord(c->ev_start, c->stream));
   if (preset) HIP_TRY(hipStreamWaitEvent(c->stream, c->ev_alt, 0));   // inside the timed span
-  HIP_TRY(launch_mbfs_setup<OffT>(a, static_cast<MbfsArgs<OffT>*>(c->b_args), setup_grid,
+  BatchSources src{};
+  std::memcpy(src.v, sources, nsrc * sizeof(int32_t));
+  HIP_TRY(launch_mbfs_setup<OffT>(a, static_cast<MbfsArgs<OffT>*>(c->b_args), src, setup_grid,
                                   c->stream));
   c->b_last_args_off64 = g->off64;
   std::memcpy(c->b_last_args, &a, sizeof a);
@@ -2092,9 +2079,10 @@ static int batch_stats(pbbs_ctx* c, pbbs_bfs_stats* stats) {
 }
 
 template <typename OffT>
-static int run_batch(pbbs_ctx* c, pbbs_graph* g, int32_t nsrc, int32_t* d_parent, int32_t* d_depth,
+static int run_batch(pbbs_ctx* c, pbbs_graph* g, const int32_t* sources, int32_t nsrc,
+                     int32_t* d_parent, int32_t* d_depth,
                      bool own_out, pbbs_bfs_stats* stats) {
-  int rc = begin_batch<OffT>(c, g, nsrc, d_parent, d_depth, own_out);
+  int rc = begin_batch<OffT>(c, g, sources, nsrc, d_parent, d_depth, own_out);
   bool done = false;
   while (rc == PBBS_OK && !done) rc = poll_run(c, true, &done);
   if (rc != PBBS_OK) return rc;
@@ -2128,10 +2116,8 @@ extern "C" int pbbs_bfs_batch(pbbs_ctx* c, pbbs_graph* g, const int32_t* sources
   if (rc != PBBS_OK) return rc;
   // outputs to the caller's device buffers only when both are given
   const bool own_out = !(dev_out && parents && depths);
-  HIP_TRY(hipMemcpyAsync(c->b_sources, sources, nsrc * sizeof(int32_t), hipMemcpyHostToDevice,
-                         c->stream));
-  rc = g->off64 ? run_batch<int64_t>(c, g, nsrc, parents, depths, own_out, stats)
-                : run_batch<uint32_t>(c, g, nsrc, parents, depths, own_out, stats);
+  rc = g->off64 ? run_batch<int64_t>(c, g, sources, nsrc, parents, depths, own_out, stats)
+                : run_batch<uint32_t>(c, g, sources, nsrc, parents, depths, own_out, stats);
   if (rc != PBBS_OK) return rc;
   int32_t* dp = own_out ? c->b_parent : parents;
   int32_t* dd = own_out ? c->b_depth : depths;
@@ -2275,10 +2261,8 @@ int async_begin(pbbs_ctx* c, pbbs_graph* g, const int32_t* sources, int32_t nsrc
   if (!g->symmetric) return fail(PBBS_ERR_INVALID, "batched BFS needs a symmetric graph");
   rc = ensure_batch_workspace(c, g->n, (int64_t)nsrc * g->n, true);
   if (rc != PBBS_OK) return rc;
-  HIP_TRY(hipMemcpyAsync(c->b_sources, sources, nsrc * sizeof(int32_t), hipMemcpyHostToDevice,
-                         c->stream));
-  return g->off64 ? begin_batch<int64_t>(c, g, nsrc, nullptr, nullptr, true)
-                  : begin_batch<uint32_t>(c, g, nsrc, nullptr, nullptr, true);
+  return g->off64 ? begin_batch<int64_t>(c, g, sources, nsrc, nullptr, nullptr, true)
+                  : begin_batch<uint32_t>(c, g, sources, nsrc, nullptr, nullptr, true);
 }
 
 int async_poll(pbbs_ctx* c, bool* done) { return poll_run(c, false, done); }
