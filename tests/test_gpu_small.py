@@ -55,7 +55,6 @@ CASES = {
 
 @pytest.mark.parametrize("wide", [False, True])
 def test_small_graphs(ctx, wide):
-    import torch
     jobs = []
     for name, make in CASES.items():
         g = make()
@@ -67,10 +66,11 @@ def test_small_graphs(ctx, wide):
             assert np.array_equal(p, wp) and np.array_equal(d, wd), (name, s)
             assert st["reached"] == (wd < g.n).sum() and st["levels"] == wd[wd < g.n].max() + 1
             assert st["edges_reached"] == g.degrees()[wd < g.n].sum()
-            out = [torch.empty(g.n, dtype=torch.int32, device="cuda") for _ in range(2)]
-            dg.bfs_device(s, out[0].data_ptr(), out[1].data_ptr())
-            assert np.array_equal(out[0].cpu().numpy(), wp), (name, s)
-            assert np.array_equal(out[1].cpu().numpy(), wd), (name, s)
+            st = dg.bfs_device(s)
+            r = dg.check_device(s, *ctx.outputs())
+            assert r["valid"] == 1 and r["depth_bad"] == 0, (name, s, r)
+            assert r["max_rule_bad"] in ((0,) if dg.info["sorted"] else (0, -1)), (name, s, r)
+            assert r["reached"] == st["reached"]
             if s == g.n - 1:
                 jobs.append((name, dg, s, wp, wd))
     # several graphs: with the two past the limits, and without
