@@ -67,10 +67,10 @@ def test_small_graphs(ctx, wide):
             assert st["reached"] == (wd < g.n).sum() and st["levels"] == wd[wd < g.n].max() + 1
             assert st["edges_reached"] == g.degrees()[wd < g.n].sum()
             st = dg.bfs_device(s)
-            r = dg.check_device(s, *ctx.outputs())
-            assert r["valid"] == 1 and r["depth_bad"] == 0, (name, s, r)
-            assert r["max_rule_bad"] in ((0,) if dg.info["sorted"] else (0, -1)), (name, s, r)
-            assert r["reached"] == st["reached"]
+            assert st["reached"] == (wd < g.n).sum()
+            if dg.info["symmetric"]:   # the checker's rules read rows as in-neighbours
+                r = dg.check_device(s, *ctx.outputs())
+                assert r["valid"] == 1 and r["max_rule_bad"] == 0 and r["depth_bad"] == 0, (name, r)
             if s == g.n - 1:
                 jobs.append((name, dg, s, wp, wd))
     # several graphs: with the two past the limits, and without
