@@ -339,8 +339,8 @@ def run_single(args):
         },
         "roofline": {
             "bound": "hbm",
-            "kernel": ("one BFS: bfs_init_kernel + one bfs_persist_kernel launch running every "
-                       "level" if st["launches"] == 1 else
+            "kernel": ("one BFS: every level in one launch (bfs_deep_kernel, then its parents, "
+                       "or bfs_persist_kernel or bfs_small_kernel)" if st["launches"] == 1 else
                        "one BFS launch sequence (bfs_init_kernel + bfs_level_kernel per level)"),
             "launches_per_bfs": st["launches"],
             "achieved": round(B / (event_ms / 1e3) / 1e9, 1),
@@ -772,7 +772,7 @@ def mis_traffic():
 
 
 def st_traffic():
-    """HBM bytes per forest of the reserve and commit steps, from the committed
+    """HBM bytes per forest of the reserve, commit and tree steps, from the committed
     FETCH_SIZE / WRITE_SIZE summary (profiles/traffic_st_rmat24e.json)."""
     path = os.path.join(ROOT, "profiles", "traffic_st_rmat24e.json")
     if not os.path.exists(path):
@@ -780,7 +780,8 @@ def st_traffic():
     with open(path) as f:
         t = json.load(f)
     return (t["reserve_fetch_bytes_per_forest"] + t["reserve_write_bytes_per_forest"] +
-            t["commit_fetch_bytes_per_forest"] + t["commit_write_bytes_per_forest"])
+            t["commit_fetch_bytes_per_forest"] + t["commit_write_bytes_per_forest"] +
+            t["tree_fetch_bytes_per_forest"] + t["tree_write_bytes_per_forest"])
 
 
 MIS_GRAPH = ("rMatGraph_JR_12_16000000 (one of the three graphs the maximal independent set "
@@ -900,7 +901,7 @@ def run_st(args):
         "rounds": int(st["rounds"]), "forest_edges": int(cnt),
         "medges_per_s": round(u.size / (ev / 1e3) / 1e6, 1),
         "roofline": {
-            "bound": "hbm", "kernel": "st_reserve + st_commit + st_schedule + st_pack per round",
+            "bound": "hbm", "kernel": "st_reserve + st_commit per round, st_tree at some",
             "achieved": round(Bst / (ev / 1e3) / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(Bst / (ev / 1e3) / 1e9 / HBM_PEAK_GBS, 4),
             "algorithmic_bytes": Bst,
