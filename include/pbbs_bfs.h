@@ -90,11 +90,14 @@ typedef struct {
                                the rest in the frontier bitmap only, and the level after it
                                expands that bitmap (same outputs, bounded workspace) */
     int32_t persist;        /* 1 = a single-source BFS runs every level in one persistent
-                               launch whose workgroups (grid_blocks, else one per CU) meet at
+                               launch whose workgroups (grid_blocks, else one per CU or, on
+                               those smaller graphs, per 1024 vertices) meet at
                                a grid barrier between levels; one such launch per device at a
                                time, others run one level per launch.  0 = one level per
                                launch.  2 (default) = persistent once the graph's previous run
-                               needed 64 levels or more (deep graphs), else one per launch.
+                               needed 64 levels or more (deep graphs) or the graph has at most
+                               2^17 vertices and 2^23 entries (48 to 96 workgroups), else one
+                               per launch.
                                With 1, and with 2 from 16 levels, symmetric graphs of rows of
                                at most 64 entries meet every few levels instead (deterministic
                                runs).  With 2 and grid_blocks 0, graphs of up to 16384 vertices

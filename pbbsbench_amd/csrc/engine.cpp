@@ -1125,13 +1125,27 @@ static int persist_capacity(pbbs_ctx* c, bool off64, int variant) {
   return std::min(per_cu * c->num_cus, kMaxGrid);
 }
 
-// Workgroups of a persistent launch: the tuning's grid_blocks if set, else
-// one per CU (on the 216^3 torus, 325 levels: 6.97 ms on 256 workgroups,
-// 7.87 on 128, 8.77 on 512, 13.9 on 1024; the barrier's cost grows with
-// the workgroups that meet at it); never more than fit at once.
-static int persist_grid(pbbs_ctx* c, int cap) {
+// Graphs whose levels are short enough for a few workgroups: what a level costs
+// is then its launch or its barrier, and a barrier of 48 to 96 workgroups is
+// the cheaper one.  us a search, one level per launch against persistent, rMat:
+// n 2^14, m 228K 83 against 82; 2^16, 494K 110 / 93, 1.8M 101 / 86, 6.2M 96 /
+// 88; 2^17, 3.7M 112 / 100; randlocal 100K, 984K 126 / 113.  Past the line: rMat
+// 2^18, 3.9M 120 / 114, 14.5M 113 / 115; randlocal 300K, 5.8M 123 / 135; rMat
+// 2^19, 15.5M 129 / 154.
+constexpr int64_t kFewMaxN = int64_t(1) << 17;
+constexpr int64_t kFewMaxM = int64_t(1) << 23;
+static bool few_groups(const pbbs_graph* g) { return g->n <= kFewMaxN && g->m <= kFewMaxM; }
+
+// Workgroups of a persistent launch: the tuning's grid_blocks if set, else one
+// per 1024 vertices, 48 to 96 (n 2^16: 48 workgroups 94-87 us, 64 86, 96 87,
+// 192 95; 2^17: 64 102, 96 100, 192 107), and one per CU on larger graphs (the
+// 216^3 torus, 325 levels: 6.97 ms on 256 workgroups, 7.87 on 128, 8.77 on
+// 512, 13.9 on 1024; the barrier's cost grows with the workgroups that meet at
+// it); never more than fit at once.
+static int persist_grid(pbbs_ctx* c, const pbbs_graph* g, int cap) {
   const int want = c->tuning.grid_blocks > 0 ? std::min(c->tuning.grid_blocks, kMaxGrid)
-                                             : c->num_cus;
+                   : few_groups(g) ? (int)std::min<int64_t>(96, std::max<int64_t>(48, g->n / 1024))
+                                   : c->num_cus;
   return std::min(want, cap);
 }
 
@@ -1139,12 +1153,15 @@ static int persist_grid(pbbs_ctx* c, int cap) {
 // previous single-source run needed at least this many levels: there the
 // per-level launch and drain cost dominates (C3, 325 levels: 6.97 ms
 // persistent against 9.36 ms one launch per level), while shallow graphs
-// run faster one launch per level (C4: 0.53 against 0.79 ms).
+// run faster one launch per level (C4: 0.53 against 0.79 ms).  Graphs of
+// few_groups take it whatever their depth, where the context's own workspace
+// is used and the grid is left open.
 constexpr int kPersistMinLevels = 64;
 
-static bool want_persist(const pbbs_ctx* c, const pbbs_graph* g) {
+static bool want_persist(const pbbs_ctx* c, const pbbs_graph* g, bool own) {
   if (c->tuning.persist == 1) return true;
   if (c->tuning.persist != 2) return false;
+  if (own && few_groups(g) && c->tuning.grid_blocks == 0) return true;
   return g->last_launches[0] - 1 >= kPersistMinLevels;   // levels + 1 launches
 }
 
@@ -1224,11 +1241,11 @@ static int begin_bfs(pbbs_ctx* c, pbbs_graph* g, int32_t s, int32_t* d_parent, i
       grid = dg;
     }
   }
-  if (allow_persist && !persist && want_persist(c, g)) {
+  if (allow_persist && !persist && want_persist(c, g, own)) {
     const int cap = persist_capacity(c, g->off64, variant);
     if (cap >= 1 && take_persist(c)) {
       persist = true;
-      grid = persist_grid(c, cap);
+      grid = persist_grid(c, g, cap);
     }
   }
   if (!persist) {
@@ -1353,14 +1370,15 @@ static int32_t* ensure_pinned(pbbs_ctx* c, int64_t entries) {
   return c->p_out;
 }
 
-// Graphs one workgroup searches faster than the device does with a launch per
-// level.  The line is where device-output calls meet, workgroup against
-// launches: rMat 2^12 vertices, 53K edges 64 against 84 us; 2^13, 59K 70
-// against 91; 2^12, 100K 84 against 77; 2^13, 110K 98 against 87; torus 18^3,
-// 35K 81 against 105; 24^3, 83K 131 against 125.  (Host outputs gain 40 us
-// more: the kernel writes them to pinned memory.)  Only where the tuning leaves
-// the launch shape open (a set grid or persist mode asks for the level
-// kernels); any-parent runs keep their directions, which decide their parents.
+// Graphs one workgroup searches faster than more do, with a barrier or a launch
+// per level.  The line is where device-output calls meet, one workgroup against
+// the better of the two: rMat 2^12 vertices, 53K edges 57 against 75 us; 2^13,
+// 72K 71 against 77; 2^14, 62K 74 against 94; 2^12, 100K 84 against 77; 2^13,
+// 110K 98 against 87; torus 18^3, 35K 81 against 105; 24^3, 83K 131 against 125.
+// (Host outputs gain 50 us more: the kernel writes them to pinned memory.)  Only
+// where the tuning leaves the launch shape open (a set grid or persist mode asks
+// for the level kernels); any-parent runs keep their directions, which decide
+// their parents.
 constexpr int64_t kSmallMaxM = 80000;
 static bool want_small(const pbbs_ctx* c, const pbbs_graph* g, bool any_parent) {
   return !any_parent && g->n <= kSmallMaxN && g->m <= kSmallMaxM && c->tuning.persist == 2 &&
@@ -1821,8 +1839,8 @@ static int prepare_graph(pbbs_ctx* c, pbbs_graph* g, uint32_t what) {
     if (rc != PBBS_OK) return rc;
     // and for the grid of a persistent launch
     const int cap = persist_capacity(c, g->off64, variant);
-    if (cap >= 1 && persist_grid(c, cap) != grid) {
-      rc = ensure_bounds(c, g, (int64_t)persist_grid(c, cap) * kWavesPerBlock, &bounds);
+    if (cap >= 1 && persist_grid(c, g, cap) != grid) {
+      rc = ensure_bounds(c, g, (int64_t)persist_grid(c, g, cap) * kWavesPerBlock, &bounds);
       if (rc != PBBS_OK) return rc;
     }
   }
