@@ -1126,25 +1126,28 @@ static int persist_capacity(pbbs_ctx* c, bool off64, int variant) {
 }
 
 // Graphs whose levels are short enough for a few workgroups: what a level costs
-// is then its launch or its barrier, and a barrier of 48 to 96 workgroups is
+// is then its launch or its barrier, and a barrier of 48 to 128 workgroups is
 // the cheaper one.  us a search, one level per launch against persistent, rMat:
 // n 2^14, m 228K 83 against 82; 2^16, 494K 110 / 93, 1.8M 101 / 86, 6.2M 96 /
-// 88; 2^17, 3.7M 112 / 100; randlocal 100K, 984K 126 / 113.  Past the line: rMat
-// 2^18, 3.9M 120 / 114, 14.5M 113 / 115; randlocal 300K, 5.8M 123 / 135; rMat
-// 2^19, 15.5M 129 / 154.
-constexpr int64_t kFewMaxN = int64_t(1) << 17;
-constexpr int64_t kFewMaxM = int64_t(1) << 23;
-static bool few_groups(const pbbs_graph* g) { return g->n <= kFewMaxN && g->m <= kFewMaxM; }
+// 88; 2^17, 3.7M 112 / 100; 2^18, 1.5M 129 / 115, 3.9M 120 / 111; randlocal 100K,
+// 984K 126 / 113; 200K, 2.0M 137 / 122; 260K, 4.1M 122 / 117.  Past the line:
+// rMat 2^18, 7.6M 116 / 113, 14.5M 113 / 115; randlocal 300K, 5.8M 123 / 132;
+// rMat 2^19, 15.5M 129 / 141.
+constexpr int64_t kFewMaxN = int64_t(1) << 18;
+constexpr int64_t kFewMaxM = int64_t(1) << 22;   // twice as many up to half as many vertices
+static bool few_groups(const pbbs_graph* g) {
+  return g->n <= kFewMaxN && g->m <= (g->n <= kFewMaxN / 2 ? 2 * kFewMaxM : kFewMaxM);
+}
 
 // Workgroups of a persistent launch: the tuning's grid_blocks if set, else one
-// per 1024 vertices, 48 to 96 (n 2^16: 48 workgroups 94-87 us, 64 86, 96 87,
-// 192 95; 2^17: 64 102, 96 100, 192 107), and one per CU on larger graphs (the
-// 216^3 torus, 325 levels: 6.97 ms on 256 workgroups, 7.87 on 128, 8.77 on
+// per 1024 vertices, 48 to 128 (n 2^16: 48 workgroups 87 us, 64 86, 96 87, 192
+// 95; 2^17: 64 102, 96 100, 128 101, 192 107; 2^18, 3.9M: 96 116, 128 111, 192
+// 114), and one per CU on larger graphs (the 216^3 torus, 325 levels: 6.97 ms on 256 workgroups, 7.87 on 128, 8.77 on
 // 512, 13.9 on 1024; the barrier's cost grows with the workgroups that meet at
 // it); never more than fit at once.
 static int persist_grid(pbbs_ctx* c, const pbbs_graph* g, int cap) {
   const int want = c->tuning.grid_blocks > 0 ? std::min(c->tuning.grid_blocks, kMaxGrid)
-                   : few_groups(g) ? (int)std::min<int64_t>(96, std::max<int64_t>(48, g->n / 1024))
+                   : few_groups(g) ? (int)std::min<int64_t>(128, std::max<int64_t>(48, g->n / 1024))
                                    : c->num_cus;
   return std::min(want, cap);
 }

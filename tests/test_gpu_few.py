@@ -28,8 +28,10 @@ def reversed_rows(g):
 CASES = {
     "fewest": lambda: random_graph(16385, 9_000, 1),
     "one workgroup's edges and more": lambda: random_graph(3_000, 90_000, 2),
-    "most vertices": lambda: random_graph(1 << 17, 700_000, 3),
-    "past most vertices": lambda: random_graph((1 << 17) + 1, 700_000, 4),
+    "half of the most vertices": lambda: random_graph(1 << 17, 700_000, 3),
+    "past half of the most vertices": lambda: random_graph((1 << 17) + 1, 700_000, 4),
+    "most vertices": lambda: random_graph(1 << 18, 600_000, 9),
+    "past most vertices": lambda: random_graph((1 << 18) + 1, 600_000, 10),
     "dense": lambda: random_graph(20_000, 2_000_000, 5),
     "directed": lambda: random_graph(60_001, 400_000, 6, directed=True),
     "reversed rows": lambda: reversed_rows(random_graph(60_001, 400_000, 7)),
