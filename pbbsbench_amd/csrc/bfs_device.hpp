@@ -91,6 +91,11 @@ constexpr long long kStreamMinM = 1ll << 26;
 // (rMat 2^24, 15M edges: 884 us; 2^22, 4.5M: 257), so they meet at a 48th of m;
 // the line is at m / (kStreamTd * td_to_bu_div), a 40th by default.
 constexpr unsigned kStreamTd = 2;
+// The more edges F_k has, the sooner the general bottom-up level finds a parent,
+// while streaming costs the same (and 8 us in the next level): rMat 2^22, 128M
+// entries, F_2 of 11.7M edges 224 + 49 us general and 190 + 57 streamed, of 15.0M
+// 170 + 45 and 205 + 54.  The line is at a 10th of m.
+constexpr unsigned kStreamBu = 10;
 
 // Everything a level kernel needs.  The init kernel copies it into device
 // memory so one captured HIP graph of level launches serves every run that

@@ -1144,12 +1144,13 @@ __device__ __forceinline__ int level_mode(const BfsArgs<OffT>& A, int prev, unsi
 }
 
 // Whether bu_stream takes the level: F_k is small and known by its queue (the
-// level before was top-down), and top-down would take longer.
+// level before was top-down), and both the top-down and the general bottom-up
+// level would take longer.
 template <typename OffT>
 __device__ __forceinline__ bool stream_level(const BfsArgs<OffT>& A, int prev,
                                              unsigned long long cnt, unsigned long long E) {
   return prev == kTopDown && A.symmetric && A.td_to_bu_div > 0 && cnt <= kStreamMax &&
-         A.m >= kStreamMinM &&
+         A.m >= kStreamMinM && E * kStreamBu <= (unsigned long long)A.m &&
          E * (unsigned)A.td_to_bu_div * kStreamTd > (unsigned long long)A.m;
 }
 
