@@ -71,8 +71,7 @@ struct BfsState {
 // and any-parent levels (bottom-up rows probed from their smallest entry up,
 // the first frontier neighbour found taken as the parent, sorted or not).
 // kLevelStream: sorted rows with records, on graphs where a small frontier of
-// hubs may meet most of the edges (levels that stream the adjacency; kept out of
-// the other variants, whose levels they slow by 1 to 2%).
+// hubs may have many edges (levels that stream the adjacency).
 enum LevelVariant {
   kLevelUnsorted = 0,
   kLevelSorted = 1,
@@ -96,6 +95,10 @@ constexpr unsigned kStreamTd = 2;
 // entries, F_2 of 11.7M edges 224 + 49 us general and 190 + 57 streamed, of 15.0M
 // 170 + 45 and 205 + 54.  The line is at a 10th of m.
 constexpr unsigned kStreamBu = 10;
+// Levels that may stream, from the source's on: a small frontier with many edges
+// is the first or second ring of neighbours.  The others run in the plain
+// kernel, which starts 0.2 us sooner.
+constexpr int kStreamLevels = 4;
 
 // Everything a level kernel needs.  The init kernel copies it into device
 // memory so one captured HIP graph of level launches serves every run that
@@ -133,6 +136,7 @@ struct BfsArgs {
   int32_t symmetric;
   int32_t num_cus;             // CUs of the device (workgroup slot = blockIdx / num_cus)
   int32_t small_rows;          // 1 if no row has more than 64 entries (top-down slices by entry)
+  int64_t stream_min, stream_max;  // a streaming level's edges: more than, at most
   unsigned long long* deep_words;  // meeting words of a deep launch to clear, or null
   long long wait_ticks;        // persistent launch: longest barrier wait (device wall-clock
                                // ticks) before the launch gives up

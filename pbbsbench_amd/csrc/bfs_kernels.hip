@@ -1144,14 +1144,12 @@ __device__ __forceinline__ int level_mode(const BfsArgs<OffT>& A, int prev, unsi
 }
 
 // Whether bu_stream takes the level: F_k is small and known by its queue (the
-// level before was top-down), and both the top-down and the general bottom-up
-// level would take longer.
-template <typename OffT>
-__device__ __forceinline__ bool stream_level(const BfsArgs<OffT>& A, int prev,
-                                             unsigned long long cnt, unsigned long long E) {
-  return prev == kTopDown && A.symmetric && A.td_to_bu_div > 0 && cnt <= kStreamMax &&
-         A.m >= kStreamMinM && E * kStreamBu <= (unsigned long long)A.m &&
-         E * (unsigned)A.td_to_bu_div * kStreamTd > (unsigned long long)A.m;
+// level before was top-down), and its edges lie in (lo, hi], where both the
+// top-down and the general bottom-up level would take longer.
+__device__ __forceinline__ bool stream_level(int prev, bool qover, unsigned long long cnt,
+                                             unsigned long long E, unsigned long long lo,
+                                             unsigned long long hi) {
+  return (prev == kTopDown) & !qover & (cnt <= kStreamMax) & (E > lo) & (E <= hi);
 }
 
 // Level k of the BFS, as workgroup vb of a grid of vg workgroups (the
@@ -1212,61 +1210,15 @@ __device__ void rebuild_bitmaps(const BfsArgs<OffT>* __restrict__ A, const int k
   }
 }
 
-template <typename OffT, bool kSorted, bool kTops, bool kLazy = false, bool kAsc = false,
-          bool kStream = false>
-__device__ __forceinline__ bool level_step(const BfsArgs<OffT>* __restrict__ A, const int k,
-                                           StageBuf& sb, BuLds<OffT>& bl, const unsigned vb,
-                                           const unsigned vg, LazyBitmaps* lz = nullptr) {
+// What a level does besides its expansion: workgroup 0's bookkeeping, and the
+// bitmaps.  Args: a pointer to the argument block, in any address space.
+template <typename Args>
+__device__ __forceinline__ void level_open(const Args A, const int k, const int mode,
+                                           const unsigned long long cnt,
+                                           const unsigned long long E, const unsigned vb,
+                                           const unsigned vg, const bool keep) {
   BfsState* st = A->st;
-  const int c0 = k % 3, c1 = (k + 1) % 3, c2 = (k + 2) % 3;
-  unsigned long long cnt = 0, E = 0;
-  unsigned long long qc[kSubQueues];   // F_k's sub-queue counters, kept for the expansion
-#pragma unroll
-  for (int s = 0; s < kSubQueues; ++s) {
-    qc[s] = st->ctr[c0][s];
-    cnt += (uint32_t)qc[s];
-    E += qc[s] >> 32;
-  }
-  if (cnt == 0) {
-    // F_k has no vertex to expand: the BFS is over.  The first kernel to see
-    // it closes the books; later (overshoot) launches return at once.
-    if (vb == 0 && threadIdx.x == 0 && !st->finished) {
-      const uint32_t z = st->d0[c0];
-      st->reached += z;
-      if (z) st->max_depth = k;
-      st->finished = 1;
-      BfsState* hst = A->host_state;   // the host reads these once host_status[0] is set
-      hst->reached = st->reached;
-      hst->edges_reached = st->edges_reached;
-      hst->max_depth = st->max_depth;
-      hst->td_levels = st->td_levels;
-      hst->bu_levels = st->bu_levels;
-      __threadfence_system();
-      __hip_atomic_store(&A->host_status[1], k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      __hip_atomic_store(&A->host_status[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-    return false;
-  }
-  const int prev = k == 0 ? kTopDown : st->modes[(k - 1) & 3];
-  int mode = level_mode(*A, prev, cnt, E);
-  const bool qover = st->qover[c0] != 0;
-  bool stream = false;
-  if constexpr (kStream) {
-    stream = stream_level(*A, prev, cnt, E) && !qover;
-    if (stream) mode = kBottomUp;
-  }
-  bool keep = true;   // this level keeps the bitmaps
-  if constexpr (kLazy) {
-    if (lz->on) {
-      if (mode == kBottomUp || qover) {
-        rebuild_bitmaps(A, k, vb, vg);
-        if (!grid_barrier(st, A->host_status, A->wait_ticks, *lz->bv)) return false;
-        lz->on = false;
-      } else {
-        keep = false;
-      }
-    }
-  }
+  const int c0 = k % 3, c2 = (k + 2) % 3;
   if (vb == 0 && threadIdx.x == 0) {
     st->modes[k & 3] = mode;
     st->reached += cnt + st->d0[c0];
@@ -1302,6 +1254,15 @@ __device__ __forceinline__ bool level_step(const BfsArgs<OffT>* __restrict__ A, 
       }
     }
   }
+}
+
+// What the expansion of level k reads and writes.
+template <typename OffT, bool kTops, typename Args>
+__device__ __forceinline__ LevelView<OffT> level_view(const Args A, const int k, const bool keep,
+                                                      const int prev, const unsigned vb,
+                                                      const unsigned vg) {
+  BfsState* st = A->st;
+  const int c0 = k % 3, c1 = (k + 1) % 3;
   const int sq = (int)(vb % kSubQueues);
   LevelView<OffT> a;
   a.off = glob(A->off);
@@ -1334,6 +1295,83 @@ __device__ __forceinline__ bool level_step(const BfsArgs<OffT>* __restrict__ A, 
   a.W = (long long)vg * kWavesPerBlock;
   a.k = k;
   a.serial_depth = A->bu_serial_depth;
+  return a;
+}
+
+template <typename OffT, bool kSorted, bool kTops, bool kLazy = false, bool kAsc = false,
+          bool kStream = false>
+__device__ __forceinline__ bool level_step(const BfsArgs<OffT>* __restrict__ A, const int k,
+                                           StageBuf& sb, BuLds<OffT>& bl, const unsigned vb,
+                                           const unsigned vg, LazyBitmaps* lz = nullptr) {
+  BfsState* st = A->st;
+  const int c0 = k % 3;
+  unsigned long long cnt = 0, E = 0;
+  unsigned long long qc[kSubQueues];   // F_k's sub-queue counters, kept for the expansion
+#pragma unroll
+  for (int s = 0; s < kSubQueues; ++s) {
+    qc[s] = st->ctr[c0][s];
+    cnt += (uint32_t)qc[s];
+    E += qc[s] >> 32;
+  }
+  const int prev = k == 0 ? kTopDown : st->modes[(k - 1) & 3];
+  const bool qover = st->qover[c0] != 0;
+  if (cnt == 0) {
+    // F_k has no vertex to expand: the BFS is over.  The first kernel to see
+    // it closes the books; later (overshoot) launches return at once.
+    if (vb == 0 && threadIdx.x == 0 && !st->finished) {
+      const uint32_t z = st->d0[c0];
+      st->reached += z;
+      if (z) st->max_depth = k;
+      st->finished = 1;
+      BfsState* hst = A->host_state;   // the host reads these once host_status[0] is set
+      hst->reached = st->reached;
+      hst->edges_reached = st->edges_reached;
+      hst->max_depth = st->max_depth;
+      hst->td_levels = st->td_levels;
+      hst->bu_levels = st->bu_levels;
+      __threadfence_system();
+      __hip_atomic_store(&A->host_status[1], k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(&A->host_status[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    return false;
+  }
+  const int mode = level_mode(*A, prev, cnt, E);
+  if constexpr (kStream) {
+    if (__builtin_expect(stream_level(prev, qover, cnt, E, A->stream_min, A->stream_max), 0)) {
+      // The streamed level on its own: scalars it shared with the other kinds
+      // would stay in registers through them, and what they spill costs each of
+      // their passes.  So it reads the argument block again, through a pointer
+      // that the compiler does not know to be A (from the kernel's arguments).
+      typedef const __attribute__((address_space(4))) BfsArgs<OffT>* ConstArgs;
+      const ConstArgs B = *(const __attribute__((address_space(4))) ConstArgs*)
+          __builtin_amdgcn_kernarg_segment_ptr();
+      int kk = __builtin_amdgcn_readfirstlane(k);
+      unsigned vb2 = vb, vg2 = vg;
+      asm("" : "+s"(kk), "+s"(vb2), "+s"(vg2));
+      level_open(B, kk, kBottomUp, cnt, E, vb2, vg2, true);
+      const LevelView<OffT> a = level_view<OffT, kTops>(B, kk, true, kTopDown, vb2, vg2);
+      Stage stg;
+      slot_priority(B->num_cus);
+      bu_stream(a, sb, stg, bl, qc);
+      __builtin_amdgcn_s_setprio(0);
+      stage_flush_block(a, sb, stg, false);
+      return true;
+    }
+  }
+  bool keep = true;   // this level keeps the bitmaps
+  if constexpr (kLazy) {
+    if (lz->on) {
+      if (mode == kBottomUp || qover) {
+        rebuild_bitmaps(A, k, vb, vg);
+        if (!grid_barrier(st, A->host_status, A->wait_ticks, *lz->bv)) return false;
+        lz->on = false;
+      } else {
+        keep = false;
+      }
+    }
+  }
+  level_open(A, k, mode, cnt, E, vb, vg, keep);
+  const LevelView<OffT> a = level_view<OffT, kTops>(A, k, keep, prev, vb, vg);
   Stage stg;
   if (mode == kTopDown) {
     if (prev == kBottomUp || qover)
@@ -1343,10 +1381,14 @@ __device__ __forceinline__ bool level_step(const BfsArgs<OffT>* __restrict__ A, 
   } else
   {
     slot_priority(A->num_cus);   // bottom-up only: top-down levels measured the same with it
-    if (kStream && stream)
-      bu_stream(a, sb, stg, bl, qc);
-    else
-      bottom_up<OffT, kSorted, kTops, kAsc>(a, sb, stg, bl);
+    LevelView<OffT> b = a;
+    if constexpr (kStream) {
+      // in vector registers: the streamed level's code leaves this kernel short
+      // of scalar ones (25 reloads of spilled scalars a pass without, 3 with)
+      asm("" : "+v"(b.parent), "+v"(b.depth), "+v"(b.fb_next), "+v"(b.visited), "+v"(b.adj),
+               "+v"(b.tops));
+    }
+    bottom_up<OffT, kSorted, kTops, kAsc>(b, sb, stg, bl);
     __builtin_amdgcn_s_setprio(0);
   }
   stage_flush_block(a, sb, stg, mode == kTopDown);
@@ -2588,6 +2630,7 @@ __global__ __launch_bounds__(kBlock) void graph_offsets_kernel(
     const OffT* __restrict__ off, long long n, long long m, long long nwords,
     unsigned long long* __restrict__ iso, unsigned long long* __restrict__ counters) {
   const unsigned lane = lane_id();
+  unsigned long long squares = 0;   // of the degrees; at most max degree * m < 2^63
   for (long long b = global_wave(); b < nwords; b += num_waves()) {
     const long long v = b * kWave + lane;
     bool isolated = false, bad = false;
@@ -2598,6 +2641,7 @@ __global__ __launch_bounds__(kBlock) void graph_offsets_kernel(
       if (!bad) {
         deg = (unsigned long long)(o1 - o0);
         isolated = deg == 0;
+        squares += deg * deg;
       }
     }
     const unsigned long long im = __ballot(isolated);
@@ -2615,6 +2659,9 @@ __global__ __launch_bounds__(kBlock) void graph_offsets_kernel(
       if (bm) atomicAdd(&counters[2], (unsigned long long)__popcll(bm));
     }
   }
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) squares += __shfl_xor(squares, d);
+  if (lane == 0 && squares) atomicAdd(&counters[7], squares);
 }
 
 // Pass 2 (offsets validated: 0 = off[0] <= ... <= off[n] = m).

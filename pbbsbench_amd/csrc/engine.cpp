@@ -297,6 +297,7 @@ struct pbbs_graph {
   int64_t nrows = 0;
   int64_t isolated = 0;
   int64_t max_degree = 0;
+  double met_degree = 0;                 // sum of squared degrees / m
   int64_t device_bytes = 0;
   // Level launches the last single-source [0] / batched [1] run needed (its
   // levels plus the launch that found the frontier empty); 0 = none yet.
@@ -640,6 +641,7 @@ static int upload_checks(pbbs_ctx* c, pbbs_graph* g, uint32_t flags) {
     }
     g->isolated = (int64_t)h[0];
     g->max_degree = (int64_t)h[1];
+    g->met_degree = g->m > 0 ? (double)h[7] / (double)g->m : 0.0;
     g->sorted = h[4] == h[3];
     if (flags & PBBS_GRAPH_ASSUME_SYMMETRIC) {
       g->symmetric = true;
@@ -776,9 +778,17 @@ static int level_grid(pbbs_ctx* c, bool off64, int variant) {
   return std::min(per_cu * c->num_cus, kMaxGrid);
 }
 
+// The variant that launch `level` of a run takes.
+static int variant_at(int variant, int64_t level) {
+  return variant == kLevelStream && level >= kStreamLevels ? (int)kLevelSortedTops : variant;
+}
+
+// K level launches from launch `first` of a run on, as a graph.
 template <typename OffT>
-static int get_level_graph(pbbs_ctx* c, int variant, int grid, int K, hipGraphExec_t* out) {
-  const auto key = std::make_tuple((int)sizeof(OffT), variant, grid, K);
+static int get_level_graph(pbbs_ctx* c, int variant, int64_t first, int grid, int K,
+                           hipGraphExec_t* out) {
+  const int from = variant == kLevelStream ? (int)std::min<int64_t>(first, kStreamLevels) : 0;
+  const auto key = std::make_tuple((int)sizeof(OffT) * 16 + from, variant, grid, K);
   auto it = c->level_graphs.find(key);
   if (it != c->level_graphs.end()) {
     *out = it->second;
@@ -788,8 +798,8 @@ static int get_level_graph(pbbs_ctx* c, int variant, int grid, int K, hipGraphEx
   HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   hipError_t le = hipSuccess;
   for (int i = 0; i < K && le == hipSuccess; ++i)
-    le = launch_bfs_level<OffT>(static_cast<const BfsArgs<OffT>*>(c->w_args), variant, grid,
-                                c->stream);
+    le = launch_bfs_level<OffT>(static_cast<const BfsArgs<OffT>*>(c->w_args),
+                                variant_at(variant, from + i), grid, c->stream);
   const hipError_t ce = hipStreamEndCapture(c->stream, &graph);
   if (le != hipSuccess || ce != hipSuccess) {
     if (graph) (void)hipGraphDestroy(graph);
@@ -984,6 +994,8 @@ static BfsArgs<OffT> make_args(pbbs_ctx* c, pbbs_graph* g, const SingleWs& ws, i
   a.symmetric = g->symmetric ? 1 : 0;
   a.num_cus = c->num_cus;
   a.small_rows = g->max_degree <= kWave ? 1 : 0;
+  a.stream_min = a.td_to_bu_div > 0 ? a.m / ((int64_t)a.td_to_bu_div * kStreamTd) : a.m;
+  a.stream_max = a.m / kStreamBu;
   a.wait_ticks = (long long)c->tuning.persist_wait_us * c->wall_khz / 1000;
   return a;
 }
@@ -1003,8 +1015,8 @@ static int launch_chunk(pbbs_ctx* c) {
     hipGraphExec_t exec = nullptr;
     int rc;
     if (r.kind == 0)
-      rc = r.off64 ? get_level_graph<int64_t>(c, r.sorted, r.grid, r.K, &exec)
-                   : get_level_graph<uint32_t>(c, r.sorted, r.grid, r.K, &exec);
+      rc = r.off64 ? get_level_graph<int64_t>(c, r.sorted, r.launched, r.grid, r.K, &exec)
+                   : get_level_graph<uint32_t>(c, r.sorted, r.launched, r.grid, r.K, &exec);
     else
       rc = r.off64 ? get_batch_graph<int64_t>(c, r.sorted, r.grid, r.K, &exec)
                    : get_batch_graph<uint32_t>(c, r.sorted, r.grid, r.K, &exec);
@@ -1015,10 +1027,12 @@ static int launch_chunk(pbbs_ctx* c) {
       if (r.kind == 0) {
         if (r.off64)
           HIP_TRY(launch_bfs_level<int64_t>(static_cast<const BfsArgs<int64_t>*>(r.ws.args),
-                                            r.sorted, r.grid, c->stream));
+                                            variant_at(r.sorted, r.launched + i), r.grid,
+                                            c->stream));
         else
           HIP_TRY(launch_bfs_level<uint32_t>(static_cast<const BfsArgs<uint32_t>*>(r.ws.args),
-                                             r.sorted, r.grid, c->stream));
+                                             variant_at(r.sorted, r.launched + i), r.grid,
+                                             c->stream));
       } else {
         if (r.off64)
           HIP_TRY(launch_mbfs_level<int64_t>(static_cast<const MbfsArgs<int64_t>*>(c->b_args),
@@ -1106,11 +1120,18 @@ static int level_variant(const pbbs_graph* g, const uint32_t* tops) {
 }
 
 // The variant of a run with a launch per level: streaming levels where
-// kStreamMax vertices can have the edges that start one.
+// kStreamMax vertices can have the edges that start one.  A vertex met along an
+// edge has sum(degree^2) / m edges on average, and the rule asks for m /
+// (kStreamMax * kStreamTd * td_to_bu_div): rMat 2^22, a=.57, has 3938 for 392,
+// 2^24 6849 for 1589; rMat 2^24, a=.55, 461 for 1623 and 2^22, a=.5, 74 for 403,
+// and their searches do without the streaming kernel (600 -> 588 us at a=.5).
+// Searches of the others that meet no such level: 2^24, int64 offsets, 582 us in
+// either kernel; 2^22 and 2^23, uint32, 257 and 436 without it, 263 and 445 with
+// it (the first bottom-up level is 3% longer).
 static int launch_variant(const pbbs_ctx* c, const pbbs_graph* g, int variant) {
   const bool stream = variant == kLevelSortedTops && g->symmetric && g->m >= kStreamMinM &&
                       c->tuning.td_to_bu_div > 0 &&
-                      (double)kStreamMax * g->max_degree * kStreamTd * c->tuning.td_to_bu_div >
+                      (double)kStreamMax * g->met_degree * kStreamTd * c->tuning.td_to_bu_div >
                           (double)g->m;
   return stream ? (int)kLevelStream : variant;
 }
@@ -1285,7 +1306,7 @@ static int begin_bfs(pbbs_ctx* c, pbbs_graph* g, int32_t s, int32_t* d_parent, i
   r.graphs = own;
   if (c->tuning.use_graphs && own && !persist) {  // capture (first use only) while the stream is idle
     hipGraphExec_t exec = nullptr;
-    rc = get_level_graph<OffT>(c, variant, grid, r.K, &exec);
+    rc = get_level_graph<OffT>(c, variant, 0, grid, r.K, &exec);
     if (rc != PBBS_OK) return rc;
   }
   volatile int32_t* hs = c->host_status;
@@ -1774,8 +1795,8 @@ static int run_profile(pbbs_ctx* c, pbbs_graph* g, int32_t s, pbbs_level_profile
     hipEvent_t prev = e1;
     for (int64_t k = 0; k <= g->n + 1; ++k) {
       hipEvent_t e = new_event();
-      if (!e || launch_bfs_level<OffT>(static_cast<const BfsArgs<OffT>*>(c->w_args), variant,
-                                       grid, c->stream) != hipSuccess ||
+      if (!e || launch_bfs_level<OffT>(static_cast<const BfsArgs<OffT>*>(c->w_args),
+                                       variant_at(variant, k), grid, c->stream) != hipSuccess ||
           hipEventRecord(e, c->stream) != hipSuccess || hipEventSynchronize(e) != hipSuccess) {
         rc = fail(PBBS_ERR_HIP, "level launch failed");
         break;
@@ -2376,6 +2397,8 @@ static BfsArgs<OffT> job_args(pbbs_ctx* c, pbbs_graph* g, const JobLayout& L, un
   a.symmetric = g->symmetric ? 1 : 0;
   a.num_cus = c->num_cus;
   a.small_rows = g->max_degree <= kWave ? 1 : 0;
+  a.stream_min = a.td_to_bu_div > 0 ? a.m / ((int64_t)a.td_to_bu_div * kStreamTd) : a.m;
+  a.stream_max = a.m / kStreamBu;
   a.wait_ticks = (long long)c->tuning.persist_wait_us * c->wall_khz / 1000;
   return a;
 }

@@ -57,3 +57,23 @@ def test_range(ctx, graph):
             assert mode == "TD"
             general += 1
     assert streamed and general, found
+
+
+@pytest.mark.parametrize("graphs", [0, 1])
+@pytest.mark.parametrize("chunk", [1, 2, 3, 4, 5])
+def test_chunks(ctx, graph, chunk, graphs):
+    t = ctx.tuning
+    usual = {k: getattr(t, k) for k in ("chunk_levels", "use_graphs")}
+    dg = ctx.gen_rmat(21, 2 ** 26, 0.57, 0.19, 0.19, seed=3)   # no run yet: chunks from the first
+    try:
+        ctx.set_tuning(chunk_levels=chunk, use_graphs=graphs)
+        for s in list(small_frontiers(ctx, graph))[:2] + [0]:
+            print("[case] chunk", chunk, "graphs", graphs, "source", s, flush=True)
+            for _ in range(2):
+                st = dg.bfs_device(s)
+                r = dg.check_device(s, *ctx.outputs())
+                assert r["valid"] == 1 and r["max_rule_bad"] == 0 and r["depth_bad"] == 0, r
+                assert r["reached"] == st["reached"] and r["max_level"] + 1 == st["levels"]
+    finally:
+        ctx.set_tuning(**usual)
+        dg.free()
