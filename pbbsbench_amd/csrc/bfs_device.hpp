@@ -258,7 +258,7 @@ constexpr int kMisStripes = 64;
 constexpr int kMisMaxChunk = 1024;   // list entries one wavefront takes at a time
 constexpr int kMisPer = 4;           // fresh vertices a lane looks at together
 constexpr int kMisRetry = 1;         // second looks at a list chunk's deferred vertices
-constexpr int kMisSmall = 16384;     // vertices up to which one workgroup runs it all
+constexpr int kMisSmall = 16384;     // vertices one workgroup's states hold
 constexpr int kMisSmallBlock = 1024;
 constexpr int kAdjPad = 4;           // entries past a graph's last that may be read
 

@@ -1496,6 +1496,26 @@ extern "C" int pbbs_bfs(pbbs_ctx* c, pbbs_graph* g, int32_t source, int32_t* par
 // end any run; more means a fault, reported as an error.
 constexpr int kMisTail = 4;
 
+// Graphs whose set one workgroup finds faster than rounds over the device do.
+// What it takes grows with the vertices and entries (4.4 ns and 0.17 ns each on
+// relabelled rMat graphs) where the rounds' latency does not.  us a call, one
+// workgroup against rounds: rMat 2^14, 184K entries 99 / 103, 242K 104 / 108,
+// 300K 106 / 95, 466K 152 / 107, 1.08M 191 / 117; 2^13, 326K 99 / 100, 512K 107 /
+// 102; random graphs of 12000 vertices, 359K 97 / 101, 479K 121 / 108.  Ids in the
+// order of a local graph make long chains, which only one workgroup runs through
+// fast: random-local 16000 vertices, 306K 674 / 1840, 590K 1174 / 3930; so graphs
+// without hubs take it to more entries (16384 vertices at random, 491K: 130 / 154,
+// 655K: 148 / 121).
+constexpr int64_t kMisSmallCost = 700000;    // entries, and kMisSmallVertex for a vertex
+constexpr int64_t kMisSmallVertex = 26;
+constexpr int64_t kMisSmallEntries = 600000; // of graphs whose rows are short
+constexpr int64_t kMisSmallRow = 128;
+static bool want_small_mis(const pbbs_graph* g) {
+  return g->n <= kMisSmall &&
+         (kMisSmallVertex * g->n + g->m <= kMisSmallCost ||
+          (g->max_degree <= kMisSmallRow && g->m <= kMisSmallEntries));
+}
+
 template <typename OffT>
 static int run_mis(pbbs_ctx* c, pbbs_graph* g, int32_t* d_out, pbbs_mis_stats* stats) {
   MisArgs<OffT> a{};
@@ -1537,7 +1557,7 @@ static int run_mis(pbbs_ctx* c, pbbs_graph* g, int32_t* d_out, pbbs_mis_stats* s
   while (mis_block_start(a.block, g->n, blocks) < g->n) ++blocks;
   volatile int32_t* hs = c->host_status;
   HIP_TRY(hipEventRecord(c->ev_start, c->stream));
-  const bool small = g->n <= kMisSmall;
+  const bool small = want_small_mis(g);
   if (small) {
     HIP_TRY(launch_mis_small<OffT>(a, d_out, c->stream));
     HIP_TRY(hipEventRecord(c->ev_end, c->stream));

@@ -541,12 +541,12 @@ __global__ __launch_bounds__(kBlock) void mis_count_kernel(MisArgs<OffT> a, int 
   }
 }
 
-// Graphs of at most kMisSmall vertices: the whole run in one workgroup and one
-// launch, the states in LDS.  Vertices go 1024 at a time in id order, one per
+// Small graphs (at most kMisSmall vertices): the whole run in one workgroup and
+// one launch, the states in LDS.  Vertices go 1024 at a time in id order, one per
 // thread; all of them look until all are decided (every lower block is), then
 // the next ones, whose row bounds and first entries were loaded meanwhile.
 // Launches and round trips are all that counts here: 2^12 vertices of an RMAT
-// graph 124 -> 52 us a call, 2^14 145 -> 137, a 20^3 torus 123 -> 51.
+// graph 124 -> 52 us a call, a 20^3 torus 123 -> 51.
 template <typename OffT>
 __global__ __launch_bounds__(kMisSmallBlock) void mis_small_kernel(MisArgs<OffT> a,
                                                                    int32_t* flags_out) {
