@@ -1489,11 +1489,15 @@ extern "C" int pbbs_bfs(pbbs_ctx* c, pbbs_graph* g, int32_t source, int32_t* par
 // ------------------------------------------------- maximal independent set
 // The first chunk covers the blocks of fresh vertices and kMisTail rounds more
 // (the relabelled benchmark graphs need 3 after their last block), with the
-// output launched behind it, so that most runs meet the host once; a run that
-// is not over by then goes on in chunks of 8, and writes its output again.  A
-// round decides at least the lowest undecided vertex (its lower neighbours
-// were all decided before the round began), so n + 1 rounds past the blocks
-// end any run; more means a fault, reported as an error.
+// output launched behind it, so that most runs meet the host once; the output
+// kernels leave at once if a run is not over by then.  Three chunks of 8 more
+// rounds do the same (dense graphs need some of them: 2^16 vertices, 40 draws
+// each, 203 us, 239 with 16 rounds and the output apart).  Past those the ids make
+// long chains: chunks of a quarter of the rounds so far, 16 at least, and one
+// output pass at the end (a path of 17000 vertices 59 ms, 77 with an output pass
+// behind every 8 rounds).  A round decides at least the lowest undecided vertex
+// (its lower neighbours were all decided before the round began), so n + 1 rounds
+// past the blocks end any run; more means a fault, reported as an error.
 constexpr int kMisTail = 4;
 
 // Graphs whose set one workgroup finds faster than rounds over the device do.
@@ -1506,8 +1510,8 @@ constexpr int kMisTail = 4;
 // fast: random-local 16000 vertices, 306K 674 / 1840, 590K 1174 / 3930; so graphs
 // without hubs take it to more entries (16384 vertices at random, 491K: 130 / 154,
 // 655K: 148 / 121).
-constexpr int64_t kMisSmallCost = 700000;    // entries, and kMisSmallVertex for a vertex
-constexpr int64_t kMisSmallVertex = 26;
+constexpr int64_t kMisSmallCost = 770000;    // entries, and kMisSmallVertex for a vertex
+constexpr int64_t kMisSmallVertex = 30;
 constexpr int64_t kMisSmallEntries = 600000; // of graphs whose rows are short
 constexpr int64_t kMisSmallRow = 128;
 static bool want_small_mis(const pbbs_graph* g) {
@@ -1567,15 +1571,24 @@ static int run_mis(pbbs_ctx* c, pbbs_graph* g, int32_t* d_out, pbbs_mis_stats* s
   }
   const int64_t limit = g->n + 2 + blocks;
   int64_t launched = 0;
-  for (int64_t K = blocks + kMisTail; !small; K = 8) {
-    const int k = (int)std::min<int64_t>(K, limit - launched);
+  int64_t K = blocks + kMisTail;
+  for (int chunk = 0; !small; ++chunk) {
+    const bool short_run = chunk <= 3;
+    const int k = (int)std::min<int64_t>({K, limit - launched, 1024});
     for (int i = 0; i < k; ++i) HIP_TRY(launch_mis_round<OffT>(a, step, grid, c->stream));
     launched += k;
-    HIP_TRY(launch_mis_output<OffT>(a, d_out, pass_grid, c->stream));
+    K = chunk < 3 ? 8 : std::max<int64_t>(16, launched / 4);
+    if (short_run) HIP_TRY(launch_mis_output<OffT>(a, d_out, pass_grid, c->stream));
     HIP_TRY(hipEventRecord(c->ev_end, c->stream));
     HIP_TRY(hipEventSynchronize(c->ev_end));
     if (hs[2]) return fail(PBBS_ERR_STATE, "set worklist region overflow");
-    if (hs[0]) break;
+    if (hs[0]) {
+      if (short_run) break;
+      HIP_TRY(launch_mis_output<OffT>(a, d_out, pass_grid, c->stream));
+      HIP_TRY(hipEventRecord(c->ev_end, c->stream));
+      HIP_TRY(hipEventSynchronize(c->ev_end));
+      break;
+    }
     if (launched >= limit)
       return fail(PBBS_ERR_STATE, "set rounds did not finish in %lld launches",
                   (long long)launched);

@@ -491,10 +491,11 @@ __global__ __launch_bounds__(kBlock) void mis_init_kernel(MisArgs<OffT> a) {
 
 // Output in the reference's format (MISTime.C:38-43: one int per vertex, 1 in
 // the set, 2 not), four vertices per thread, and each workgroup's count of
-// set members in part[blockIdx.x].
+// set members in part[blockIdx.x].  Nothing before the run is over.
 template <typename OffT>
 __global__ __launch_bounds__(kBlock) void mis_output_kernel(MisArgs<OffT> a, int32_t* flags_out) {
   __shared__ unsigned wsum[kWavesPerBlock];
+  if (!*a.finished) return;
   const long long tid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   const long long nth = (long long)gridDim.x * blockDim.x;
   const long long n4 = a.n / 4;
@@ -528,6 +529,7 @@ __global__ __launch_bounds__(kBlock) void mis_output_kernel(MisArgs<OffT> a, int
 template <typename OffT>
 __global__ __launch_bounds__(kBlock) void mis_count_kernel(MisArgs<OffT> a, int parts) {
   __shared__ unsigned long long wsum[kWavesPerBlock];
+  if (!*a.finished) return;
   unsigned long long c = 0;
   for (int i = threadIdx.x; i < parts; i += kBlock) c += a.part[i];
   for (int d = 32; d >= 1; d >>= 1) c += __shfl_xor(c, d);

@@ -32,14 +32,14 @@ def rows_of(longest, n=9000, m=599_000):
 
 
 CASES = {
-    "cost at the line": lambda: exact(1000, 700_000 - 26 * 1000),
-    "cost past it": lambda: exact(1000, 700_001 - 26 * 1000),
+    "cost at the line": lambda: exact(1000, 770_000 - 30 * 1000),
+    "cost past it": lambda: exact(1000, 770_001 - 30 * 1000),
     "short rows, most entries": lambda: exact(16384, 600_000),
     "short rows, one entry more": lambda: exact(16384, 600_001),
     "most vertices and one": lambda: exact(16385, 100_000),
     "longest short row": lambda: rows_of(128),
     "a longer row": lambda: rows_of(129),
-    "few vertices, dense": lambda: exact(520, 800_000 // 520 * 520),
+    "few vertices, dense": lambda: exact(520, 900_000 // 520 * 520),
 }
 
 
