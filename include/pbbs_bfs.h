@@ -95,9 +95,12 @@ typedef struct {
                                a grid barrier between levels; one such launch per device at a
                                time, others run one level per launch.  0 = one level per
                                launch.  2 (default) = persistent once the graph's previous run
-                               needed 64 levels or more (deep graphs) or the graph has at most
-                               2^17 vertices and 2^23 entries, or 2^18 and 2^22 (48 to 128
-                               workgroups), else one per launch.
+                               needed 64 levels or more (deep graphs) or, with grid_blocks 0,
+                               the graph has at most 2^17 vertices and 2^23 entries, or 2^18
+                               and 2^22 (48 to 128 workgroups; where every level is top-down
+                               at most 2^17 vertices of 6 entries on average, and up to 16384
+                               vertices while runs need fewer than 13 levels), else one per
+                               launch.
                                With 1, and with 2 from 16 levels, symmetric graphs of rows of
                                at most 64 entries meet every few levels instead (deterministic
                                runs).  With 2 and grid_blocks 0, graphs of up to 16384 vertices

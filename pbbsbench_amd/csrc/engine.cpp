@@ -1160,12 +1160,30 @@ static bool few_groups(const pbbs_graph* g) {
   return g->n <= kFewMaxN && g->m <= (g->n <= kFewMaxN / 2 ? 2 * kFewMaxM : kFewMaxM);
 }
 
+// Of those, the searches that take it by themselves.  Not where every level is
+// top-down and wide, which a few workgroups expand too slowly (directed graphs
+// at random, 2 entries a vertex 325 / 262, 5 161 / 157, 10 133 / 148 and 20 119 /
+// 181 at 60K vertices; 200K with 5: 200 / 204); nor where many levels meet a small
+// graph, whose launches are as short as the barriers (any-parent searches of tori:
+// 8^3, 13 levels, 125 / 130; 16^3 210 / 219; 24^3, 37 levels, 327 / 341; 28^3 397 /
+// 388; rMat of 2^10 to 2^14 vertices, 5 to 10 levels, 0 to 12% faster).
+constexpr int64_t kFewTopDownN = int64_t(1) << 17;
+constexpr int64_t kFewTopDownDeg = 6;
+constexpr int64_t kFewDeepN = 16384;    // vertices from which the levels do not count
+constexpr int kFewLevels = 13;
+static bool want_few(const pbbs_ctx* c, const pbbs_graph* g) {
+  if (!few_groups(g) || c->tuning.grid_blocks != 0) return false;
+  if (!g->symmetric || c->tuning.td_to_bu_div == 0)
+    return g->n <= kFewTopDownN && g->m <= kFewTopDownDeg * g->n;
+  return g->n > kFewDeepN || g->last_launches[0] - 1 < kFewLevels;
+}
+
 // Workgroups of a persistent launch: the tuning's grid_blocks if set, else one
 // per 1024 vertices, 48 to 128 (n 2^16: 48 workgroups 87 us, 64 86, 96 87, 192
 // 95; 2^17: 64 102, 96 100, 128 101, 192 107; 2^18, 3.9M: 96 116, 128 111, 192
-// 114), and one per CU on larger graphs (the 216^3 torus, 325 levels: 6.97 ms on 256 workgroups, 7.87 on 128, 8.77 on
-// 512, 13.9 on 1024; the barrier's cost grows with the workgroups that meet at
-// it); never more than fit at once.
+// 114), and one per CU on larger graphs (the 216^3 torus, 325 levels: 6.97 ms on
+// 256 workgroups, 7.87 on 128, 8.77 on 512, 13.9 on 1024; the barrier's cost
+// grows with the workgroups that meet at it); never more than fit at once.
 static int persist_grid(pbbs_ctx* c, const pbbs_graph* g, int cap) {
   const int want = c->tuning.grid_blocks > 0 ? std::min(c->tuning.grid_blocks, kMaxGrid)
                    : few_groups(g) ? (int)std::min<int64_t>(128, std::max<int64_t>(48, g->n / 1024))
@@ -1177,15 +1195,14 @@ static int persist_grid(pbbs_ctx* c, const pbbs_graph* g, int cap) {
 // previous single-source run needed at least this many levels: there the
 // per-level launch and drain cost dominates (C3, 325 levels: 6.97 ms
 // persistent against 9.36 ms one launch per level), while shallow graphs
-// run faster one launch per level (C4: 0.53 against 0.79 ms).  Graphs of
-// few_groups take it whatever their depth, where the context's own workspace
-// is used and the grid is left open.
+// run faster one launch per level (C4: 0.53 against 0.79 ms).  Smaller graphs
+// (want_few) take it too, where the context's own workspace is used.
 constexpr int kPersistMinLevels = 64;
 
 static bool want_persist(const pbbs_ctx* c, const pbbs_graph* g, bool own) {
   if (c->tuning.persist == 1) return true;
   if (c->tuning.persist != 2) return false;
-  if (own && few_groups(g) && c->tuning.grid_blocks == 0) return true;
+  if (own && want_few(c, g)) return true;
   return g->last_launches[0] - 1 >= kPersistMinLevels;   // levels + 1 launches
 }
 
