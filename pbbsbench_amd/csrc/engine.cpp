@@ -2453,10 +2453,13 @@ static BfsArgs<OffT> job_args(pbbs_ctx* c, pbbs_graph* g, const JobLayout& L, un
   return a;
 }
 
-// Workgroups per job: proportional to n + m (at least one each, at most one
-// per 65536 edges: 16 graphs of scales 10-17 take 476 us a call with one per
-// 4096, 410 with one per 32768 to 65536, 516 with one per 131072),
-// within cap in total.
+// Workgroups per job: proportional to n + m, within cap in total, at least one each,
+// and at most one per 65536 edges or per 3072 vertices, whichever are more.  Edges:
+// 16 graphs of scales 10-17 take 476 us a call with one per 4096, 410 with one per
+// 32768 to 65536, 516 with one per 131072.  Vertices, where rows are short: 4 tori
+// of 16^3 to 40^3, by edges alone 1078 us, and with one per 8192, 4096, 3072 and 2048
+// vertices 936, 740, 705, 681; directed graphs of 30K, 60K and 100K vertices 591, 525,
+// 402, 349, 306; 4 RMAT graphs of 2^17 vertices 367, 368, 369, 369, 389.
 static void split_grid(const std::vector<pbbs_graph*>& gs, int cap, std::vector<uint32_t>& wg) {
   const size_t J = gs.size();
   double total = 0;
@@ -2465,7 +2468,8 @@ static void split_grid(const std::vector<pbbs_graph*>& gs, int cap, std::vector<
   int64_t sum = 0;
   for (size_t j = 0; j < J; ++j) {
     const int64_t share = (int64_t)((double)cap * (double)(gs[j]->n + gs[j]->m) / total);
-    const int64_t most = std::max<int64_t>(1, (gs[j]->m + 65535) / 65536);
+    const int64_t most =
+        std::max<int64_t>({1, (gs[j]->m + 65535) / 65536, gs[j]->n / 3072});
     w[j] = std::max<int64_t>(1, std::min(share, most));
     sum += w[j];
   }
