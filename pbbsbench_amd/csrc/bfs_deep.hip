@@ -250,7 +250,8 @@ __global__ __launch_bounds__(kDeepBlock) void bfs_deep_kernel(const BfsArgs<OffT
     growth = T > before ? log2f((float)T / (float)before) / (float)max(s.adv, 1u) : 0.f;
     k += (int)s.adv;
     const int bad = s.bad;
-    // bottom-up levels are due: by entries, a lower bound on the edges too
+    // bottom-up levels are due, by an estimate: T is about |F|, more by vertices
+    // claimed at too large a depth, and each has an edge at least
     const bool big = A.td_to_bu_div > 0 &&
                      (unsigned long long)T * 2 > (unsigned long long)A.m / (unsigned)A.td_to_bu_div &&
                      T > (unsigned)kDeepSolo;

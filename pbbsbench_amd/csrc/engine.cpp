@@ -194,6 +194,7 @@ struct pbbs_ctx {
     int64_t launched = 0;
     int64_t limit = 0;
     bool persist = false;    // single source: every level in one persistent launch
+    uint64_t deep_key = 0;   // of a deep launch: how large frontiers may get
     bool token = false;      // holds the device's persistent-launch token
     bool any_parent = false; // single source: PBBS_BFS_ANY_PARENT levels
     int32_t source = 0;
@@ -302,8 +303,9 @@ struct pbbs_graph {
   // Level launches the last single-source [0] / batched [1] run needed (its
   // levels plus the launch that found the frontier empty); 0 = none yet.
   std::atomic<int> last_launches[2] = {0, 0};
-  // A deep launch found the graph's frontiers too large for it: not tried again.
-  std::atomic<bool> not_deep{false};
+  // The last deep launch that found the graph's frontiers too large for it, by
+  // what decides that (deep_key); 0 = none.  Not tried again in that form.
+  std::atomic<uint64_t> deep_refused{0};
 };
 
 // One persistent launch per device at a time: its grid fills the device and
@@ -1085,7 +1087,7 @@ static int poll_run_impl(pbbs_ctx* c, bool wait, bool* done) {
     r.persist = false;
     if (!c->host_status[2])
       return fail(PBBS_ERR_STATE, "persistent BFS launch ended before the BFS did");
-    if (c->host_status[2] == 2) r.graph->not_deep = true;
+    if (c->host_status[2] == 2) r.graph->deep_refused = r.deep_key;
     // the launch gave up waiting at a barrier (the device was shared), or the
     // frontier outgrew the deep path: run the BFS again from its start, one
     // level per launch
@@ -1217,8 +1219,7 @@ static bool want_persist(const pbbs_ctx* c, const pbbs_graph* g, bool own) {
 constexpr int kDeepMinLevels = 16;
 
 static bool want_deep(const pbbs_ctx* c, const pbbs_graph* g, bool own, bool any_parent) {
-  if (!own || any_parent || !g->symmetric || g->max_degree > kDeepMaxRow || g->not_deep)
-    return false;
+  if (!own || any_parent || !g->symmetric || g->max_degree > kDeepMaxRow) return false;
   if (c->tuning.persist == 1) return true;
   return c->tuning.persist == 2 && g->last_launches[0] - 1 >= kDeepMinLevels;
 }
@@ -1256,6 +1257,12 @@ static int deep_grid(pbbs_ctx* c) {
   return std::min({want, per_cu * c->num_cus, kDeepMaxGroups});
 }
 
+// What decides how large a deep launch's frontiers may get: its lists, and the
+// edges from which bottom-up levels are due.
+static uint64_t deep_key(const pbbs_ctx* c, int groups) {
+  return (uint64_t)groups << 32 | (uint32_t)c->tuning.td_to_bu_div;
+}
+
 // Starts a single-source BFS.  With allow_persist, every level runs in one
 // persistent launch when the tuning asks for it and this context can take
 // the device's token; otherwise the levels run one per launch, in captured
@@ -1277,7 +1284,8 @@ static int begin_bfs(pbbs_ctx* c, pbbs_graph* g, int32_t s, int32_t* d_parent, i
   DeepWs dws{};
   if (allow_persist && want_deep(c, g, own, any_parent)) {
     const int dg = deep_grid<OffT>(c);
-    if (dg >= 1 && ensure_deep(c, dg, &dws) && take_persist(c)) {
+    if (dg >= 1 && g->deep_refused != deep_key(c, dg) && ensure_deep(c, dg, &dws) &&
+        take_persist(c)) {
       persist = deep = true;
       grid = dg;
     }
@@ -1315,6 +1323,7 @@ static int begin_bfs(pbbs_ctx* c, pbbs_graph* g, int32_t s, int32_t* d_parent, i
   r.launched = 0;
   r.limit = g->n + 2;
   r.persist = persist;
+  r.deep_key = deep ? deep_key(c, grid) : 0;
   r.any_parent = any_parent;
   r.source = s;
   r.parent = d_parent;
