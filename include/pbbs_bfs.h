@@ -150,7 +150,9 @@ int pbbs_graph_free(pbbs_graph* g);
  * first BFS costs what a later one does and the HBM it takes is known:
  *   PBBS_PREPARE_SINGLE  the bottom-up share bounds for ctx's launch shape
  *                        and, on a sorted symmetric graph with bu_row_tops
- *                        on, the 32-byte row-top records (32 n bytes);
+ *                        on, the 32-byte row-top records (32 n bytes); for a
+ *                        symmetric graph of rows of at most 64 entries also
+ *                        ctx's lists for deep graphs (17 MB, once a context);
  *   PBBS_PREPARE_BATCH   (symmetric graphs) degree ranks, the rank-id copy
  *                        of the adjacency, the list of non-isolated rows and
  *                        the pull slices for ctx's batched launch shape

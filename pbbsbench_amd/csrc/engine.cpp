@@ -338,13 +338,17 @@ static void free_workspace(pbbs_ctx* c) {
   (void)hipFree(c->w_qe);
   c->w_parent = c->w_depth = nullptr;
   c->w_bits = nullptr;
-  (void)hipFree(c->d_deep);
-  c->d_deep = nullptr;
-  c->d_groups = 0;
   c->w_q = nullptr;
   c->w_qe = nullptr;
   c->cap_n = 0;
   c->cap_q = 0;
+}
+
+// The deep path's buffers; their size does not depend on a graph's.
+static void free_deep(pbbs_ctx* c) {
+  (void)hipFree(c->d_deep);
+  c->d_deep = nullptr;
+  c->d_groups = 0;
 }
 
 // Control words of a set run: three sets of kMisStripes region counts, one
@@ -542,6 +546,7 @@ int pbbs_ctx_destroy(pbbs_ctx* c) {
   for (auto& kv : c->level_graphs) (void)hipGraphExecDestroy(kv.second);
   for (auto& kv : c->batch_graphs) (void)hipGraphExecDestroy(kv.second);
   free_workspace(c);
+  free_deep(c);
   free_mis_workspace(c);
   free_st_workspace(c);
   (void)hipFree(c->b_masks);
@@ -1218,8 +1223,10 @@ static bool want_persist(const pbbs_ctx* c, const pbbs_graph* g, bool own) {
 // parents.
 constexpr int kDeepMinLevels = 16;
 
+static bool deep_rows(const pbbs_graph* g) { return g->symmetric && g->max_degree <= kDeepMaxRow; }
+
 static bool want_deep(const pbbs_ctx* c, const pbbs_graph* g, bool own, bool any_parent) {
-  if (!own || any_parent || !g->symmetric || g->max_degree > kDeepMaxRow) return false;
+  if (!own || any_parent || !deep_rows(g)) return false;
   if (c->tuning.persist == 1) return true;
   return c->tuning.persist == 2 && g->last_launches[0] - 1 >= kDeepMinLevels;
 }
@@ -1230,9 +1237,7 @@ static bool ensure_deep(pbbs_ctx* c, int groups, DeepWs* ws) {
   const size_t words = 2 * kDeepMaxGroups, part = 4 * kDeepMaxParts;
   const size_t lists = (size_t)2 * groups * kDeepCap;
   if (groups > c->d_groups) {
-    (void)hipFree(c->d_deep);
-    c->d_deep = nullptr;
-    c->d_groups = 0;
+    free_deep(c);
     if (hipMalloc(&c->d_deep, (words + part + lists) * sizeof(unsigned long long)) != hipSuccess) {
       (void)hipGetLastError();
       return false;
@@ -1284,10 +1289,13 @@ static int begin_bfs(pbbs_ctx* c, pbbs_graph* g, int32_t s, int32_t* d_parent, i
   DeepWs dws{};
   if (allow_persist && want_deep(c, g, own, any_parent)) {
     const int dg = deep_grid<OffT>(c);
-    if (dg >= 1 && g->deep_refused != deep_key(c, dg) && ensure_deep(c, dg, &dws) &&
-        take_persist(c)) {
-      persist = deep = true;
-      grid = dg;
+    if (dg >= 1 && g->deep_refused != deep_key(c, dg) && take_persist(c)) {
+      if (ensure_deep(c, dg, &dws)) {
+        persist = deep = true;
+        grid = dg;
+      } else {
+        release_persist(c);
+      }
     }
   }
   if (allow_persist && !persist && want_persist(c, g, own)) {
@@ -1926,6 +1934,13 @@ static int prepare_graph(pbbs_ctx* c, pbbs_graph* g, uint32_t what) {
       rc = ensure_bounds(c, g, (int64_t)persist_grid(c, g, cap) * kWavesPerBlock, &bounds);
       if (rc != PBBS_OK) return rc;
     }
+    // and the deep path's lists, which its first search would allocate (without
+    // room for them it is not taken)
+    if (deep_rows(g) && c->tuning.persist != 0 && !want_small(c, g, false)) {
+      const int dg = deep_grid<OffT>(c);
+      DeepWs ws{};
+      if (dg >= 1) (void)ensure_deep(c, dg, &ws);
+    }
   }
   if ((what & PBBS_PREPARE_BATCH) && g->symmetric) {
     int rc = ensure_ranks<OffT>(c, g);
@@ -2305,6 +2320,7 @@ void ctx_trim(pbbs_ctx* c) {
   (void)hipStreamSynchronize(c->stream);
   (void)hipStreamSynchronize(c->side);
   free_workspace(c);
+  free_deep(c);
   free_mis_workspace(c);
   free_st_workspace(c);
   (void)hipFree(c->b_masks);
