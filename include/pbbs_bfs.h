@@ -108,7 +108,9 @@ typedef struct {
     int32_t persist_wait_us;/* longest wait at a barrier of a persistent launch (default
                                200000); a launch that waits longer (its grid could not gather,
                                e.g. on a device shared with other processes) gives up and the
-                               BFS runs again one level per launch, with the same outputs */
+                               BFS runs again one level per launch, with the same outputs.
+                               With persist 2 the smaller graphs' launches (48 to 128
+                               workgroups) wait 5000 at most */
 } pbbs_tuning;
 
 int pbbs_tuning_get(const pbbs_ctx* ctx, pbbs_tuning* out);

@@ -1178,6 +1178,10 @@ constexpr int64_t kFewTopDownN = int64_t(1) << 17;
 constexpr int64_t kFewTopDownDeg = 6;
 constexpr int64_t kFewDeepN = 16384;    // vertices from which the levels do not count
 constexpr int kFewLevels = 13;
+// Their longest wait at a barrier when nobody asked for a persistent launch.  The
+// levels take some 10 us each, so a longer wait means that other work holds the
+// compute units; a launch per level then gets along with those that are left.
+constexpr int kFewWaitUs = 5000;
 static bool want_few(const pbbs_ctx* c, const pbbs_graph* g) {
   if (!few_groups(g) || c->tuning.grid_blocks != 0) return false;
   if (!g->symmetric || c->tuning.td_to_bu_div == 0)
@@ -1319,6 +1323,8 @@ static int begin_bfs(pbbs_ctx* c, pbbs_graph* g, int32_t s, int32_t* d_parent, i
   }
   BfsArgs<OffT> a = make_args<OffT>(c, g, ws, d_parent, d_depth, bounds, tops);
   a.deep_words = dws.words;
+  if (persist && !deep && c->tuning.persist == 2 && few_groups(g))
+    a.wait_ticks = std::min<long long>(a.wait_ticks, (long long)kFewWaitUs * c->wall_khz / 1000);
   const int init_grid =
       (int)std::max<int64_t>(1, std::min<int64_t>((g->n + kBlock - 1) / kBlock, c->num_cus * 16));
   pbbs_ctx::Run& r = c->run;
