@@ -2853,7 +2853,7 @@ hipError_t launch_bfs_multi(const BfsArgs<OffT>* args, const uint32_t* wg_begin,
   hipLaunchKernelGGL(bfs_multi_init_kernel<OffT>, dim3(init_grid, njobs), dim3(kBlock), 0, stream,
                      args, sources);
   const hipError_t e = hipGetLastError();
-  if (e != hipSuccess || grid == 0) return e;   // the presets alone
+  if (e != hipSuccess) return e;
   if (sorted)
     hipLaunchKernelGGL((bfs_multi_kernel<OffT, true>), dim3(grid), dim3(kBlock), 0, stream, args,
                        wg_begin, njobs);

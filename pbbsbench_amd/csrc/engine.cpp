@@ -2416,12 +2416,12 @@ static int64_t job_align(int64_t x) { return (x + kJobAlign - 1) / kJobAlign * k
 // Device memory of one single-source BFS outside the context workspace:
 // control block, per-workgroup level counters, argument block, the four
 // bitmaps, the two frontier queues and their edge prefixes (queue_cap(n,
-// queue_div) entries per sub-queue region), and optionally parent and depth.
+// queue_div) entries per sub-queue region).
 struct JobLayout {
-  int64_t st, wg, args, bits, q, qe, parent, depth, total, qcap;
+  int64_t st, wg, args, bits, q, qe, total, qcap;
 };
 
-static JobLayout job_layout_q(int64_t n, int64_t qcap, bool outputs) {
+static JobLayout job_layout_q(int64_t n, int64_t qcap) {
   JobLayout L;
   const int64_t nwords = (n + kWave - 1) / kWave;
   L.qcap = qcap;
@@ -2431,14 +2431,12 @@ static JobLayout job_layout_q(int64_t n, int64_t qcap, bool outputs) {
   L.bits = job_align(L.args + (int64_t)sizeof(BfsArgs<int64_t>));
   L.q = job_align(L.bits + 4 * nwords * (int64_t)sizeof(unsigned long long));
   L.qe = job_align(L.q + 2 * kSubQueues * L.qcap * (int64_t)sizeof(int32_t));
-  L.parent = job_align(L.qe + 2 * kSubQueues * L.qcap * (int64_t)sizeof(uint32_t));
-  L.depth = outputs ? job_align(L.parent + n * (int64_t)sizeof(int32_t)) : L.parent;
-  L.total = outputs ? job_align(L.depth + n * (int64_t)sizeof(int32_t)) : L.parent;
+  L.total = job_align(L.qe + 2 * kSubQueues * L.qcap * (int64_t)sizeof(uint32_t));
   return L;
 }
 
-static JobLayout job_layout(int64_t n, int32_t queue_div, bool outputs) {
-  return job_layout_q(n, queue_cap(n, queue_div), outputs);
+static JobLayout job_layout(int64_t n, int32_t queue_div) {
+  return job_layout_q(n, queue_cap(n, queue_div));
 }
 
 // BfsArgs of a BFS whose workspace is laid out by L at base.
@@ -2683,7 +2681,7 @@ extern "C" int pbbs_bfs_multi(pbbs_ctx* c, int32_t njobs, pbbs_graph* const* gra
   std::vector<JobLayout> L(njobs);
   std::vector<int64_t> at(njobs + 1, 0), out_at(njobs + 1, 0);
   for (int j = 0; j < njobs; ++j) {
-    L[j] = job_layout(gs[j]->n, c->tuning.queue_div, false);
+    L[j] = job_layout(gs[j]->n, c->tuning.queue_div);
     at[j + 1] = at[j] + L[j].total;
     out_at[j + 1] = out_at[j] + gs[j]->n;
   }
@@ -2817,14 +2815,14 @@ int bfs_in_block(pbbs_ctx* c, pbbs_graph* g, int32_t s, int32_t* d_parent, int32
   if (s < 0 || (int64_t)s >= g->n)
     return fail(PBBS_ERR_INVALID, "source %d outside [0, %lld)", s, (long long)g->n);
   if (!blk) return fail(PBBS_ERR_STATE, "no scratch block on device %d", c->device);
-  const int64_t fixed = job_layout_q(g->n, 0, false).total;
+  const int64_t fixed = job_layout_q(g->n, 0).total;
   const int64_t per_entry = 2 * (int64_t)kSubQueues * (sizeof(int32_t) + sizeof(uint32_t));
   const int64_t room = (bytes - fixed - 2 * kJobAlign) / per_entry;
   const int64_t qcap = std::min(queue_cap(g->n, c->tuning.queue_div), room);
   if (qcap < kWave)
     return fail(PBBS_ERR_LIMIT, "n=%lld leaves no room for the frontier queues in %lld bytes",
                 (long long)g->n, (long long)bytes);
-  const JobLayout L = job_layout_q(g->n, qcap, false);
+  const JobLayout L = job_layout_q(g->n, qcap);
   if (L.total > bytes) return fail(PBBS_ERR_LIMIT, "workspace layout exceeds the scratch block");
   SingleWs ws;
   ws.bits = reinterpret_cast<unsigned long long*>(blk + L.bits);

@@ -493,9 +493,8 @@ __global__ __launch_bounds__(kBlock) void st_any_kernel(StArgs a) {
   }
 }
 
-// filter_map of R (ST.C:67-69): per-workgroup counts of reserved entries,
-// one workgroup's scan (st_schedule_kernel's scan with `out_scan`), then the
-// ordered writes.
+// filter_map of R (ST.C:67-69): per-workgroup counts of reserved entries, one
+// workgroup's scan of them, then the ordered writes.
 __global__ __launch_bounds__(kBlock) void st_out_count_kernel(StArgs a) {
   __shared__ unsigned wsum[kWavesPerBlock];
   long long lo, hi;
