@@ -98,8 +98,9 @@ typedef struct {
                                needed 64 levels or more (deep graphs) or, with grid_blocks 0,
                                the graph has at most 2^17 vertices and 2^23 entries, or 2^18
                                and 2^22 (48 to 128 workgroups; where every level is top-down
-                               at most 2^17 vertices of 6 entries on average, and up to 16384
-                               vertices while runs need fewer than 13 levels), else one per
+                               at most 2^17 vertices of 6 entries on average; up to 16384
+                               vertices if the previous run needed fewer than 13 levels, or,
+                               with none yet, a row has more than 16 entries), else one per
                                launch.
                                With 1, and with 2 from 16 levels, symmetric graphs of rows of
                                at most 64 entries meet every few levels instead (deterministic

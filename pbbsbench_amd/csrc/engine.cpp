@@ -1173,11 +1173,13 @@ static bool few_groups(const pbbs_graph* g) {
 // 181 at 60K vertices; 200K with 5: 200 / 204); nor where many levels meet a small
 // graph, whose launches are as short as the barriers (any-parent searches of tori:
 // 8^3, 13 levels, 125 / 130; 16^3 210 / 219; 24^3, 37 levels, 327 / 341; 28^3 397 /
-// 388; rMat of 2^10 to 2^14 vertices, 5 to 10 levels, 0 to 12% faster).
+// 388; rMat of 2^10 to 2^14 vertices, 5 to 10 levels, 0 to 12% faster).  Before a
+// graph's first search its rows stand for the levels.
 constexpr int64_t kFewTopDownN = int64_t(1) << 17;
 constexpr int64_t kFewTopDownDeg = 6;
 constexpr int64_t kFewDeepN = 16384;    // vertices from which the levels do not count
 constexpr int kFewLevels = 13;
+constexpr int64_t kFewRow = 16;         // a small graph of shorter rows has many levels
 // Their longest wait at a barrier when nobody asked for a persistent launch.  The
 // levels take some 10 us each, so a longer wait means that other work holds the
 // compute units; a launch per level then gets along with those that are left.
@@ -1186,7 +1188,9 @@ static bool want_few(const pbbs_ctx* c, const pbbs_graph* g) {
   if (!few_groups(g) || c->tuning.grid_blocks != 0) return false;
   if (!g->symmetric || c->tuning.td_to_bu_div == 0)
     return g->n <= kFewTopDownN && g->m <= kFewTopDownDeg * g->n;
-  return g->n > kFewDeepN || g->last_launches[0] - 1 < kFewLevels;
+  if (g->n > kFewDeepN) return true;
+  const int launches = g->last_launches[0];   // none yet: by the rows
+  return launches ? launches - 1 < kFewLevels : g->max_degree > kFewRow;
 }
 
 // Workgroups of a persistent launch: the tuning's grid_blocks if set, else one

@@ -25,6 +25,15 @@ def uniform(n, m):
     return pb.from_edges(n, r.integers(0, n, m), r.integers(0, n, m))
 
 
+def tail(fan, length=30):
+    """A path of `length` vertices to one with a row of `fan` entries; 5 starts it."""
+    ids = np.r_[5, np.arange(6, 6 + length - 1)]
+    hub = ids[-1]
+    leaves = hub + 1 + np.arange(fan - 1)
+    return pb.from_edges(int(leaves[-1]) + 1, np.r_[ids[:-1], np.full(fan - 1, hub)],
+                         np.r_[ids[1:], leaves])
+
+
 # graph, any-parent, tuning, one launch on the first search and on the next
 CASES = {
     "directed, 6 entries a row": (lambda: directed(60_000, 360_000), False, {}, 1, 1),
@@ -35,8 +44,11 @@ CASES = {
     "no bottom-up levels": (lambda: uniform(30_000, 300_000), False, {"td_to_bu_div": 0}, 0, 0),
     "bottom-up levels": (lambda: uniform(30_000, 300_000), False, {}, 1, 1),
     "few levels": (lambda: uniform(12_000, 150_000), True, {}, 1, 1),
-    "many levels, small": (lambda: pb.grid3d(24), True, {}, 1, 0),
-    "13 levels, small": (lambda: pb.grid3d(8), True, {}, 1, 0),
+    "many levels, small": (lambda: pb.grid3d(24), True, {}, 0, 0),
+    "13 levels, small": (lambda: pb.grid3d(8), True, {}, 0, 0),
+    "many levels, a long row": (lambda: tail(16), True, {}, 0, 0),
+    "many levels, a longer row": (lambda: tail(17), True, {}, 1, 0),
+    "few levels, short rows": (lambda: tail(3, 4), True, {}, 0, 1),
     "many levels": (lambda: pb.grid3d(27), True, {}, 1, 1),
     "set grid": (lambda: uniform(30_000, 300_000), False, {"grid_blocks": 64}, 0, 0),
 }
