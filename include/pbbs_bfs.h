@@ -218,7 +218,9 @@ int pbbs_bfs_noalloc(pbbs_ctx* ctx, pbbs_graph* g, int32_t source, int32_t* pare
 
 /* ---- maximal independent set ------------------------------------------ */
 typedef struct {
-    int32_t rounds;         /* worklist rounds run (a round that found no work ends the run) */
+    int32_t rounds;         /* worklist rounds run (a round that found no work ends the run);
+                               where one workgroup ran the whole call (small graphs), its
+                               passes over undecided vertices, at least one per 1024 of n */
     int32_t pad;
     int64_t members;        /* vertices in the set */
     double  device_ms;      /* hipEvent time: init kernel start -> output written */

@@ -12,9 +12,9 @@
 // spread over the workgroup.  (A binary search per edge over the degree sums
 // made ten LDS reads of it.)  What bounds a run are its steps' waits, two
 // gathers and four barriers each: a call to device memory on rMat of 2^12
-// vertices, 53K edges takes 64 us (84 with a launch per level), on a torus of
-// 12^3 58 (86).  Eight edges a thread halve the steps of a wide level and
-// lengthen the narrow ones: 67 and 69 us.
+// vertices, 53K edges takes 54 us (69 with a launch per level), on a torus of
+// 12^3 52 (156).  Eight edges a thread halve the steps of a wide level and
+// lengthen the narrow ones: 5 and 19% more.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

@@ -1440,8 +1440,8 @@ static int32_t* ensure_pinned(pbbs_ctx* c, int64_t entries) {
 
 // Graphs one workgroup searches faster than more do, with a barrier or a launch
 // per level.  The line is where device-output calls meet, one workgroup against
-// the better of the two: rMat 2^12 vertices, 53K edges 57 against 75 us; 2^13,
-// 72K 71 against 77; 2^14, 62K 74 against 94; 2^12, 100K 84 against 77; 2^13,
+// the better of the two: rMat 2^12 vertices, 53K edges 54 against 69 us; 2^13,
+// 72K 72 against 78; 2^14, 62K 74 against 94; 2^12, 100K 84 against 77; 2^13,
 // 110K 98 against 87; torus 18^3, 35K 81 against 105; 24^3, 83K 131 against 125.
 // (Host outputs gain 50 us more: the kernel writes them to pinned memory.)  Only
 // where the tuning leaves the launch shape open (a set grid or persist mode asks

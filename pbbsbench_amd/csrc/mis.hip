@@ -295,8 +295,8 @@ __device__ __forceinline__ void mis_fresh(const MisArgs<OffT>& a, long long v0, 
 // `region` holds both.
 //
 // 2^24 vertices, 381M entries (RMAT, relabelled), a call: 1.16 ms with every
-// vertex in round 0 and byte states, 0.63 so; 256^3 torus, relabelled, 0.84 and
-// 0.51.  A block of 2.6M vertices takes about 80 us, 70% of it with the CUs'
+// vertex in round 0 and byte states, 0.58 so; 256^3 torus, relabelled, 0.84 and
+// 0.48.  A block of 2.6M vertices takes about 80 us, 70% of it with the CUs'
 // address units busy on the state gathers (one lane's address a cycle), which
 // hit the L2 at 75-78%.
 template <typename OffT, int kStep>
